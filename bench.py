@@ -45,117 +45,40 @@ def qwen3_8b_config(layers):
 
 
 class GemmTimer:
-    """Wraps the matrix-core GEMM launcher in every module that calls it: records a HIP event pair on
-    the launching stream around every GEMM of the timed region, with its algorithmic FLOPs
-    (2*M*N*K)."""
+    """Wraps the matrix-core GEMM launchers in every module that calls them: records a HIP event pair on
+    the launching stream around every GEMM of the timed region, with its algorithmic FLOPs (2*M*N*K, both
+    weights of a gate/up pair)."""
 
     def __init__(self, modules):
-        self.mods = [m for m in modules if hasattr(m, "gemm_nt_into")]
-        self.orig = self.mods[0].gemm_nt_into
-        assert all(m.gemm_nt_into is self.orig for m in self.mods)
-        # the gate/up GEMM with the SwiGLU epilogue (two weights, one launch)
-        self.gu_mods = [m for m in modules if hasattr(m, "gate_up_swiglu_into")]
-        self.gu_orig = self.gu_mods[0].gate_up_swiglu_into if self.gu_mods else None
-        # the same with Y^T stored from the epilogue too (the MLP block's forward)
-        self.gt_mods = [m for m in modules if hasattr(m, "gate_up_swiglu_t_into")]
-        self.gt_orig = self.gt_mods[0].gate_up_swiglu_t_into if self.gt_mods else None
-        # the shared-input projections (q/k/v: up to three weights, one launch)
-        self.mu_mods = [m for m in modules if hasattr(m, "gemm_nt_multi_into")]
-        self.mu_orig = self.mu_mods[0].gemm_nt_multi_into if self.mu_mods else None
-        # the projection GEMM with the residual sum in its epilogue
-        self.rs_mods = [m for m in modules if hasattr(m, "gemm_nt_residual_into")]
-        self.rs_orig = self.rs_mods[0].gemm_nt_residual_into if self.rs_mods else None
-        # the down projection's input-gradient GEMM with the SwiGLU backward epilogue
-        self.sb_mods = [m for m in modules if hasattr(m, "swiglu_bwd_gemm_into")]
-        self.sb_orig = self.sb_mods[0].swiglu_bwd_gemm_into if self.sb_mods else None
+        self.slots = [(m, name, getattr(m, name)) for m in modules for name in ("gemm", "gemm_nt_into") if hasattr(m, name)]
+        assert any(name == "gemm" for _, name, _ in self.slots)
         self.records = []
         self.active = False
 
-    def __enter__(self):
+    def _timed(self, name, orig):
         import torch
-        orig = self.orig
+        from qwen3_triton import _hip as H
 
-        def timed(a, lda, bnk, ldb, out, m, n, k, **kw):
+        def run(*args, **kw):
             if not self.active:
-                return orig(a, lda, bnk, ldb, out, m, n, k, **kw)
+                return orig(*args, **kw)
+            m, n, k = args[3:6] if name == "gemm" else args[5:8]
+            weights = 2 if kw.get("epilogue") == H.GEMM_GATE_UP else 1
             s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             s.record()
-            orig(a, lda, bnk, ldb, out, m, n, k, **kw)
+            orig(*args, **kw)
             e.record()
-            self.records.append((s, e, 2.0 * m * n * k))
+            self.records.append((s, e, 2.0 * m * n * k * weights))
+        return run
 
-        def timed_gu(x, wg, wu, g, u, y, m, n, k):
-            if not self.active:
-                return self.gu_orig(x, wg, wu, g, u, y, m, n, k)
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            self.gu_orig(x, wg, wu, g, u, y, m, n, k)
-            e.record()
-            self.records.append((s, e, 2.0 * 2 * m * n * k))
-
-        def timed_gt(x, wg, wu, g, u, y, yt, m, n, k):
-            if not self.active:
-                return self.gt_orig(x, wg, wu, g, u, y, yt, m, n, k)
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            self.gt_orig(x, wg, wu, g, u, y, yt, m, n, k)
-            e.record()
-            self.records.append((s, e, 2.0 * 2 * m * n * k))
-
-        def timed_mu(a, weights, outs, m, k):
-            if not self.active:
-                return self.mu_orig(a, weights, outs, m, k)
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            self.mu_orig(a, weights, outs, m, k)
-            e.record()
-            self.records.append((s, e, 2.0 * m * k * sum(w.shape[0] for w in weights)))
-
-        def timed_sb(dy, wt, g, u, dg, du, dgt, dut, m, n, k):
-            if not self.active:
-                return self.sb_orig(dy, wt, g, u, dg, du, dgt, dut, m, n, k)
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            self.sb_orig(dy, wt, g, u, dg, du, dgt, dut, m, n, k)
-            e.record()
-            self.records.append((s, e, 2.0 * m * n * k))
-
-        def timed_rs(a, lda, bnk, ldb, res, out, m, n, k):
-            if not self.active:
-                return self.rs_orig(a, lda, bnk, ldb, res, out, m, n, k)
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            self.rs_orig(a, lda, bnk, ldb, res, out, m, n, k)
-            e.record()
-            self.records.append((s, e, 2.0 * m * n * k))
-
-        for m in self.mods:
-            m.gemm_nt_into = timed
-        for m in self.rs_mods:
-            m.gemm_nt_residual_into = timed_rs
-        for m in self.sb_mods:
-            m.swiglu_bwd_gemm_into = timed_sb
-        for m in self.gu_mods:
-            m.gate_up_swiglu_into = timed_gu
-        for m in self.gt_mods:
-            m.gate_up_swiglu_t_into = timed_gt
-        for m in self.mu_mods:
-            m.gemm_nt_multi_into = timed_mu
+    def __enter__(self):
+        for mod, name, orig in self.slots:
+            setattr(mod, name, self._timed(name, orig))
         return self
 
     def __exit__(self, *exc):
-        for m in self.mods:
-            m.gemm_nt_into = self.orig
-        for m in self.gu_mods:
-            m.gate_up_swiglu_into = self.gu_orig
-        for m in self.gt_mods:
-            m.gate_up_swiglu_t_into = self.gt_orig
-        for m in self.mu_mods:
-            m.gemm_nt_multi_into = self.mu_orig
-        for m in self.sb_mods:
-            m.swiglu_bwd_gemm_into = self.sb_orig
-        for m in self.rs_mods:
-            m.gemm_nt_residual_into = self.rs_orig
+        for mod, name, orig in self.slots:
+            setattr(mod, name, orig)
 
     def summary(self):
         ms = sum(s.elapsed_time(e) for s, e, _ in self.records)
@@ -533,7 +456,7 @@ def main():
         "data": "synthetic (random N(0,0.02) weights, N(0,1) hidden states and upstream gradients)",
         "config": {"workload": "qwen3-8b decoder layer fwd+bwd (config #4 layer)", "model": "Qwen3-8B layer",
                    "global_batch": 4, "seq_len": 2048, "tokens_per_step": layer["tokens"], "parallelism": "none"},
-        "roofline": {"bound": "mfma", "kernel": "gemm_nt_v4_kernel (bf16 MFMA GEMM)",
+        "roofline": {"bound": "mfma", "kernel": "gemm_tile_kernel (bf16 MFMA GEMM)",
                      "achieved": round(layer["gemm_tflops"], 1), "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s",
                      "frac": round(layer["gemm_tflops"] / PEAK_BF16_TFLOPS, 4), "traffic": GEMM_TRAFFIC_BYTES_PER_LAUNCH,
                      "launches_per_step": layer["gemm_launches"] // args.steps,

@@ -244,6 +244,53 @@ int q3_gemm_swiglu_bwd(int dtype, const void* dy, int64_t lddy, const void* wt, 
 int q3_gemm_nt_multi(int dtype, const void* A, int64_t lda, int nseg, const void* const* Bs, int64_t ldb,
                      void* const* Cs, const int64_t* Ns, const int64_t* ldcs, int64_t M, int64_t K,
                      hipStream_t stream);
+/* General 16-bit matrix-core product C[m, n] = sum_k A(m, k) B(n, k) for any m, n, k (ragged ones run the
+ * same tiles; out-of-range rows and k are read as zeros), fp32 accumulation, one rounding.  Each operand is
+ * k-contiguous ([rows, k] at row stride ld) or K-major ([k, rows], a_kmajor / b_kmajor): X and a row-major W
+ * in Y = X W^T are k-contiguous, W in dX = dY W and both operands of dW = dY^T X are K-major and are read as
+ * they lie (no transposed copies).  A K-major A needs a K-major B.  Pointers 16-byte aligned, row strides
+ * and every operand's contiguous extent multiples of 8 elements, row strides below 2^22.
+ * axis / pieces: up to 3 separate matrices side by side along one axis, end[] their cumulative ends (the
+ * last is the axis' extent; the 8-element rule holds for each piece):
+ *   0  one piece: a[0], b[0], c[0]
+ *   1  along k: A = [a0 | a1 | ..], B likewise (A k-contiguous, B K-major): the input gradient of
+ *      projections sharing an input; one fp32 sum, one rounding
+ *   2  along n: b[s] -> c[s] (both k-contiguous): those projections' forward
+ *   3  along m: a[s] -> c[s] (both K-major): their weight gradients
+ * epilogue (axis 0 unless plain):
+ *   Q3_GEMM_PLAIN          C = product
+ *   Q3_GEMM_RESIDUAL       C = res + product (the product rounded first; C may be res)
+ *   Q3_GEMM_RESIDUAL_NORM  and y = C rsqrt(mean(C^2) + eps) norm_w (n <= 8192, dense C and y)
+ *   Q3_GEMM_GATE_UP        b[0], b[1] = Wg, Wu [n, k] at stride ldb[0]: C = silu(G) U from the rounded
+ *                          G = X Wg^T, U = X Wu^T, which are stored to g, u (stride ldc[0]) when given
+ *   Q3_GEMM_SWIGLU_BWD     product = dY of y = silu(g) u: c[0] = dg, c[1] = du (stride ldc[0]) from the
+ *                          inputs g, u (stride ldgu); B K-major
+ * q3_gemm_workspace_bytes: fp32 partial products of a call that splits k (0 when it does not); the workspace
+ * is caller-owned and only used during the call.
+ * Replaces: kernels/linear.py:45-105 (matmul and both backward products), kernels/mlp_precision.py:16-66. */
+enum { Q3_GEMM_PLAIN = 0, Q3_GEMM_RESIDUAL = 1, Q3_GEMM_RESIDUAL_NORM = 2, Q3_GEMM_GATE_UP = 3, Q3_GEMM_SWIGLU_BWD = 4 };
+typedef struct q3_gemm_desc {
+  int dtype, a_kmajor, b_kmajor, axis, pieces, epilogue;
+  int64_t m, n, k;
+  int64_t end[3];
+  const void* a[3];
+  int64_t lda[3];
+  const void* b[3];
+  int64_t ldb[3];
+  void* c[3];
+  int64_t ldc[3];
+  const void* res;
+  int64_t ldres;
+  const void* norm_w;
+  void* y;
+  int64_t ldy;
+  void* g;
+  void* u;
+  int64_t ldgu;
+  float eps;
+} q3_gemm_desc;
+size_t q3_gemm_workspace_bytes(const q3_gemm_desc* desc);
+int q3_gemm(const q3_gemm_desc* desc, void* workspace, size_t workspace_bytes, hipStream_t stream);
 /* Same product for arbitrary element strides: A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn];
  * any dtype (fp32 included).  SIMT path for shapes the matrix-core kernel does not take.
  * Replaces: kernels/linear.py:13-42 (_gemm with arbitrary strides). */

@@ -23,6 +23,18 @@ _i32 = ctypes.c_int
 _f32 = ctypes.c_float
 _sz = ctypes.c_size_t
 
+GEMM_PLAIN, GEMM_RESIDUAL, GEMM_RESIDUAL_NORM, GEMM_GATE_UP, GEMM_SWIGLU_BWD = range(5)
+
+
+class GemmDesc(ctypes.Structure):
+    """``q3_gemm_desc``."""
+    _fields_ = [*((n, _i32) for n in ("dtype", "a_kmajor", "b_kmajor", "axis", "pieces", "epilogue")),
+                ("m", _i64), ("n", _i64), ("k", _i64), ("end", _i64 * 3),
+                ("a", _p * 3), ("lda", _i64 * 3), ("b", _p * 3), ("ldb", _i64 * 3), ("c", _p * 3), ("ldc", _i64 * 3),
+                ("res", _p), ("ldres", _i64), ("norm_w", _p), ("y", _p), ("ldy", _i64), ("g", _p), ("u", _p),
+                ("ldgu", _i64), ("eps", _f32)]
+
+
 # name -> (restype, argtypes); mirrors include/q3hip.h one-to-one.
 SIGNATURES: dict[str, tuple] = {
     "q3_error_string": (ctypes.c_char_p, [_i32]),
@@ -100,6 +112,8 @@ SIGNATURES: dict[str, tuple] = {
     "q3_greedy_select_workspace_bytes": (_sz, [_i64]),
     "q3_greedy_select": (_i32, [_i32, _p, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _i32, _i64, _p]),
     "q3_advance": (_i32, [_p, _i64, _p]),
+    "q3_gemm_workspace_bytes": (_sz, [_p]),
+    "q3_gemm": (_i32, [_p, _p, _sz, _p]),
     "q3_gemm_strided": (_i32, [_i32, _i32, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _i64, _i64, _f32, _i32,
                                 _p]),
 }

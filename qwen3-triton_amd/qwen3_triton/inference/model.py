@@ -8,43 +8,50 @@ from pathlib import Path
 import torch
 from torch import nn
 
+from .. import _hip as H
 from .._checkpoint import read_checkpoint, resolve_tied, rope_theta
 from .._model import TritonQwen3ForCausalLM
 from ..configuration import OptimizationOptions
 from ..kernels import _ops
 from ..kernels.activation import swiglu
 from ..kernels.embedding import embedding
-from ..kernels.linear import (gemm_multi_ok, gemm_nt_multi_into, gemm_nt_residual_into, gemm_nt_residual_norm_into,
-                              gemm_residual_ok)
+from ..kernels.linear import gemm, gemm_ok
 from ..kernels.mlp_precision import gate_up_swiglu
 from ..kernels.residual import residual_add
 from . import kernels
 
 
+def _decode_rows(t, gemv):
+    """Few enough token rows for the streaming decode kernels."""
+    return gemv and t.numel() // t.shape[-1] <= kernels.DECODE_MAX_ROWS
+
+
 def _projections(h, weights, gemv):
     """[h W^T for W in weights] for a prefill chunk: one matrix-core launch over the weights side by
-    side (``q3_gemm_nt_multi``) where the shapes allow it, else one projection each."""
+    side where the operands allow it, else one projection each."""
     m, k = h.numel() // h.shape[-1], h.shape[-1]
-    if gemm_multi_ok(h, m, k, weights) and h.is_contiguous() and all(w.is_contiguous() for w in weights):
+    if not _decode_rows(h, gemv) and h.is_contiguous() and gemm_ok(h.view(m, k), *weights):
         outs = [torch.empty((*h.shape[:-1], w.shape[0]), device=h.device, dtype=h.dtype) for w in weights]
-        gemm_nt_multi_into(h.view(m, k), weights, [o.view(m, w.shape[0]) for o, w in zip(outs, weights)], m, k)
+        gemm([h.view(m, k)], weights, [o.view(m, w.shape[0]) for o, w in zip(outs, weights)], m,
+             sum(w.shape[0] for w in weights), k, axis=2)
         return outs
     return [kernels.linear(h, w, gemv=gemv) for w in weights]
 
 
 def _residual_projection(x, y, weight, gemv, norm=None):
-    """x + y W^T, the residual sum in the projection GEMM's epilogue where the shapes allow it.  With
+    """x + y W^T, the residual sum in the projection GEMM's epilogue where the operands allow it.  With
     ``norm`` (an RMSNorm module: the next block's input norm) also returns rms_norm of that sum, formed
     by the GEMM's combining pass where it has one."""
     m, k, n = y.numel() // y.shape[-1], y.shape[-1], weight.shape[0]
-    if gemm_residual_ok(y.dtype, m, n, k) and y.is_contiguous() and x.is_contiguous() and weight.is_contiguous():
+    if not _decode_rows(y, gemv) and y.is_contiguous() and x.is_contiguous() and gemm_ok(y.view(m, k), weight):
         out = torch.empty_like(x)
-        if norm is not None and n <= 8192 and norm.weight.is_contiguous() and norm.weight.dtype == x.dtype:
+        args = ([y.view(m, k)], [weight], [out.view(m, n)], m, n, k)
+        if norm is not None and n <= 8192 and n % 8 == 0 and norm.weight.is_contiguous() and \
+                norm.weight.dtype == x.dtype and norm.weight.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0:
             h = torch.empty_like(x)
-            gemm_nt_residual_norm_into(y.view(m, k), k, weight, k, x.view(m, n), out.view(m, n), norm.weight,
-                                       norm.eps, h.view(m, n), m, n, k)
+            gemm(*args, epilogue=H.GEMM_RESIDUAL_NORM, res=x.view(m, n), norm=(norm.weight, norm.eps, h.view(m, n)))
             return out, h
-        gemm_nt_residual_into(y.view(m, k), k, weight, k, x.view(m, n), out.view(m, n), m, n, k)
+        gemm(*args, epilogue=H.GEMM_RESIDUAL, res=x.view(m, n))
     else:
         out = residual_add(x, kernels.linear(y, weight, gemv=gemv))
     if norm is None:
@@ -240,8 +247,7 @@ class TritonQwen3Inference(nn.Module):
                     kernels.append(k, v, cache.keys[i], cache.values[i], start, start_dev)
                 y = kernels.attention(q, cache.keys[i], cache.values[i], start, split_decode=self.split_decode,
                                       start_dev=start_dev).reshape(b, s, -1)
-                x = _residual_projection(x, y, a.o_proj.weight, self.gemv)
-                h = kernels.rms_norm(x, layer.post_attention_layernorm.weight, layer.post_attention_layernorm.eps)
+                x, h = _residual_projection(x, y, a.o_proj.weight, self.gemv, layer.post_attention_layernorm)
                 m = layer.mlp
                 if b * s <= 8 and self.gemv:
                     y = swiglu(kernels.linear(h, m.gate_proj.weight, gemv=True),

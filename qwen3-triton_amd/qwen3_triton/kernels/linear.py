@@ -4,11 +4,12 @@ Mirrors ``qwen3_triton/kernels/linear.py:45-105``: ``matmul(a, b, *, optimized, 
 computes A[M,K] @ B[K,N] for strided matrices into a contiguous result with fp32 accumulation,
 and ``linear(x, weight)`` is Y = X W^T with dX = dY W and dW = dY^T X.
 
-Dispatch: bf16/fp16 operands go to ``q3_gemm_nt`` (MFMA), which wants both operands with K
-contiguous; an operand that is K-major only as a transposed view is first re-laid out by
-``q3_transpose`` (a bandwidth-bound copy).  fp32 or oddly strided operands use the SIMT
-``q3_gemm_strided`` kernel.  ``optimized`` is accepted for signature compatibility; the tile
-plan is fixed for gfx950.
+Dispatch: bf16/fp16 operands whose rows or columns are 16-byte chunks go to ``q3_gemm`` (matrix cores),
+which reads k-contiguous and K-major operands as they lie: X W^T, dY W and dY^T X need no transposed
+copies, whatever the token count.  Products with another output type, and layouts it does not take, go
+to ``q3_gemm_nt`` (both operands k-contiguous, after a ``q3_transpose`` copy where needed); fp32 or oddly
+strided operands use the SIMT ``q3_gemm_strided`` kernel.  ``optimized`` is accepted for signature
+compatibility; the tile plan is fixed for gfx950.
 """
 import ctypes
 
@@ -34,6 +35,65 @@ def _k_major_rows(t):
 
 def _aligned(t, ld):
     return t.data_ptr() % 16 == 0 and ld % 8 == 0
+
+
+def _ld(t):
+    """Row stride of a matrix (a single row's may be anything: its own length)."""
+    return t.stride(0) if t.shape[0] > 1 else t.shape[1]
+
+
+def _operand_ok(t):
+    """``q3_gemm``'s rule for one operand: rows of whole 16-byte chunks at a 16-byte aligned stride."""
+    ld = _ld(t)
+    return t.stride(1) == 1 and t.data_ptr() % 16 == 0 and ld % 8 == 0 and t.shape[1] % 8 == 0 and \
+        t.shape[1] <= ld < 1 << 22
+
+
+def gemm_ok(*operands):
+    """Whether ``q3_gemm`` takes these 2-D operands (each [rows, k], or [k, rows] as a K-major one)."""
+    dt, dev = operands[0].dtype, operands[0].device
+    return dt in (torch.bfloat16, torch.float16) and dev.type == 'cuda' and \
+        all(t.dtype == dt and t.device == dev and t.numel() and _operand_ok(t) for t in operands)
+
+
+def chunk_aligned(t):
+    """t, or a copy of it, contiguous and 16-byte aligned (an upstream gradient may be neither)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def gemm(a, b, c, m, n, k, *, kmajor=(False, False), axis=0, epilogue=H.GEMM_PLAIN, res=None, norm=None, g=None,
+         u=None):
+    """``q3_gemm``: c = A B over ``m x n x k``.  ``a``, ``b``, ``c`` are lists of matrices: one each, or along
+    ``axis`` (1: k, 2: n, 3: m) the pieces that lie side by side; gate/up takes both weights in ``b`` and the
+    SwiGLU backward dg and du in ``c``.  ``norm`` = (weight, eps, y) for the residual + norm epilogue."""
+    d = H.GemmDesc()
+    d.dtype, d.a_kmajor, d.b_kmajor, d.axis, d.epilogue = H.code(a[0].dtype), kmajor[0], kmajor[1], axis, epilogue
+    d.m, d.n, d.k = m, n, k
+    d.pieces = 1
+    for i, t in enumerate(a):
+        d.a[i], d.lda[i] = t.data_ptr(), _ld(t)
+    for i, t in enumerate(b):
+        d.b[i], d.ldb[i] = t.data_ptr(), _ld(t)
+    for i, t in enumerate(c):
+        d.c[i], d.ldc[i] = t.data_ptr(), _ld(t)
+    if axis:
+        parts = [t.shape[0] for t in b] if axis < 3 else [t.shape[1] for t in a]  # K-major rows are k
+        d.pieces = len(parts)
+        end = 0
+        for i, p in enumerate(parts):
+            end += p
+            d.end[i] = end
+    if res is not None:
+        d.res, d.ldres = res.data_ptr(), _ld(res)
+    if norm is not None:
+        d.norm_w, d.eps, d.y, d.ldy = norm[0].data_ptr(), float(norm[1]), norm[2].data_ptr(), _ld(norm[2])
+    if g is not None:
+        d.g, d.u, d.ldgu = g.data_ptr(), u.data_ptr(), _ld(g)
+    ref = ctypes.addressof(d)
+    nbytes = H.query("q3_gemm_workspace_bytes", ref)
+    ws = H.workspace(nbytes, a[0].device) if nbytes else None
+    H.call("q3_gemm", ref, None if ws is None else ws.data_ptr(), nbytes, H.stream())
 
 
 def gemm_nt_into(a, lda, bnk, ldb, out, m, n, k, *, alpha=1.0, accumulate=False):
@@ -81,11 +141,6 @@ def gemm_nt_residual_norm_into(a, lda, bnk, ldb, res, out, norm_w, eps, y, m, n,
            m, n, k, None if ws is None else ws.data_ptr(), ws_bytes, H.stream())
 
 
-def gemm_residual_ok(dtype, m, n, k):
-    """The fused residual epilogue serves 16-bit data in full 128 x 128 (or 256 x 256) tiles."""
-    return dtype in (torch.bfloat16, torch.float16) and m % 128 == 0 and n % 128 == 0 and k % 64 == 0
-
-
 def swiglu_bwd_gemm_into(dy, wt, g, u, dg, du, dgt, dut, m, n, k):
     """dg, du (and their transposes dgt, dut when given) of y = silu(g) * u for the upstream gradient
     dY = dy wt^T, computed in one matrix-core GEMM whose epilogue runs the SwiGLU backward
@@ -95,10 +150,6 @@ def swiglu_bwd_gemm_into(dy, wt, g, u, dg, du, dgt, dut, m, n, k):
            g.data_ptr(), u.data_ptr(), g.stride(0), dg.data_ptr(), du.data_ptr(), dg.stride(0),
            0 if dgt is None else dgt.data_ptr(), 0 if dut is None else dut.data_ptr(),
            0 if dgt is None else dgt.stride(0), m, n, k, H.stream())
-
-
-def swiglu_bwd_gemm_ok(dtype, m, n, k):
-    return dtype in (torch.bfloat16, torch.float16) and m % 256 == 0 and n % 256 == 0 and k % 64 == 0
 
 
 def gemm_nt_multi_into(a, weights, outs, m, k):
@@ -112,19 +163,16 @@ def gemm_nt_multi_into(a, weights, outs, m, k):
     H.call("q3_gemm_nt_multi", H.code(a.dtype), a.data_ptr(), k, n, bs, k, cs, ns, lds, m, k, H.stream())
 
 
-def gemm_multi_ok(x, m, k, weights):
-    """The one-launch path needs 16-bit data and full 128 x 128 (or 256 x 256) tiles."""
-    return x.dtype in (torch.bfloat16, torch.float16) and len(weights) <= 3 and m % 128 == 0 and k % 64 == 0 and \
-        all(w.shape[0] % 128 == 0 for w in weights)
-
-
-def gate_up_fused_ok(x, m, n, k):
-    return x.dtype in (torch.bfloat16, torch.float16) and m % 256 == 0 and n % 128 == 0 and k % 64 == 0
-
-
 def matmul_into(a, b, out, *, alpha=1.0, accumulate=False):
     m, k = a.shape
     n = b.shape[1]
+    if out.dtype == a.dtype and alpha == 1.0 and not accumulate and out.stride(-1) == 1:
+        # each operand k-contiguous or K-major; a K-major A needs a K-major B (dY^T X)
+        at, bt = a.stride(1) != 1, b.stride(1) == 1
+        ao, bo = a.t() if at else a, b if bt else b.t()
+        if (bt or not at) and gemm_ok(ao, bo):
+            gemm([ao], [bo], [out], m, n, k, kmajor=(at, bt))
+            return out
     if a.dtype in (torch.bfloat16, torch.float16) and k % 8 == 0:
         ar = _k_major_rows(a)
         br = _k_major_rows(b.t())
@@ -198,9 +246,9 @@ class _LinearResidual(torch.autograd.Function):
         flat = x.view(-1, x.shape[-1])
         m, k = flat.shape
         n = weight.shape[0]
-        if gemm_residual_ok(x.dtype, m, n, k) and weight.dtype == x.dtype and weight.is_contiguous():
+        if gemm_ok(flat, weight):
             out = torch.empty((m, n), device=x.device, dtype=x.dtype)
-            gemm_nt_residual_into(flat, k, weight, k, res.view(m, n), out, m, n, k)
+            gemm([flat], [weight], [out], m, n, k, epilogue=H.GEMM_RESIDUAL, res=res.view(m, n))
         else:
             out = _ops.add(res.view(m, n), matmul(flat, weight.t(), optimized=optimized))
         ctx.save_for_backward(flat, weight)
@@ -223,66 +271,43 @@ def linear_residual(x, weight, res, *, optimized=False):
 
 
 class _SharedInputProjections(torch.autograd.Function):
-    """Y_i = X W_i^T for several weights sharing one input (the q/k/v projections).  Forward runs
-    one GEMM per weight; backward packs the output gradients side by side, so dX = [dY_0 | dY_1 | ...]
-    [W_0; W_1; ...] is a single matrix-core GEMM (one rounding, no partial sums added afterwards), X is
-    transposed once, and one GEMM produces every weight gradient as a row block."""
+    """Y_i = X W_i^T for several weights sharing one input (the q/k/v projections), each direction one
+    launch over the weights side by side: the forward along n, dX = sum_i dY_i W_i along k (one fp32 sum, one
+    rounding) and the weight gradients dW_i = dY_i^T X along m."""
 
     @staticmethod
     def forward(ctx, x, *weights):
         flat = x.view(-1, x.shape[-1])
         m, k = flat.shape
-        if gemm_multi_ok(x, m, k, weights):
-            # one launch over the weights side by side (the narrow K / V projections alone would leave
-            # half of the CUs idle)
-            outs = [torch.empty((m, w.shape[0]), device=x.device, dtype=x.dtype) for w in weights]
-            gemm_nt_multi_into(flat, weights, outs, m, k)
-            outs = [o.view(*x.shape[:-1], o.shape[1]) for o in outs]
-        else:
-            outs = [matmul(flat, w.t()).view(*x.shape[:-1], w.shape[0]) for w in weights]
+        outs = [torch.empty((m, w.shape[0]), device=x.device, dtype=x.dtype) for w in weights]
+        gemm([flat], weights, outs, m, sum(w.shape[0] for w in weights), k, axis=2)
         ctx.save_for_backward(flat, *weights)
         ctx.shape = x.shape
-        return tuple(outs)
+        return tuple(o.view(*x.shape[:-1], o.shape[1]) for o in outs)
 
     @staticmethod
     def backward(ctx, *grads):
         flat, *weights = ctx.saved_tensors
         m, k = flat.shape
-        ns = [w.shape[0] for w in weights]
-        nt = sum(ns)
-        dev, dt = flat.device, flat.dtype
-        dcat = torch.empty((m, nt), device=dev, dtype=dt)
-        wt = torch.empty((k, nt), device=dev, dtype=dt)
-        col = 0
-        for gr, w, n in zip(grads, weights, ns):
-            blk = dcat[:, col:col + n]
-            if gr is None:
-                blk.zero_()
-            else:
-                _ops.copy_into(gr.contiguous().view(m, n), blk)
-            _ops.transpose_into(w, wt[:, col:col + n])
-            col += n
-        dx = torch.empty((m, k), device=dev, dtype=dt)
-        gemm_nt_into(dcat, nt, wt, nt, dx, m, k, nt)
-        dct = _ops.transpose_into(dcat, torch.empty((nt, m), device=dev, dtype=dt))
-        xt = _ops.transpose_into(flat, torch.empty((k, m), device=dev, dtype=dt))
-        dw = torch.empty((nt, k), device=dev, dtype=dt)
-        gemm_nt_into(dct, m, xt, m, dw, nt, k, m)
-        dws, row = [], 0
-        for n in ns:
-            dws.append(dw[row:row + n])
-            row += n
-        return (dx.view(ctx.shape), *dws)
+        grads = [torch.zeros((m, w.shape[0]), device=flat.device, dtype=flat.dtype) if gr is None else
+                 chunk_aligned(gr).view(m, w.shape[0]) for gr, w in zip(grads, weights)]
+        nt = sum(w.shape[0] for w in weights)
+        dx, dws = None, [None] * len(weights)
+        if ctx.needs_input_grad[0]:
+            dx = torch.empty((m, k), device=flat.device, dtype=flat.dtype)
+            gemm(grads, weights, [dx], m, k, nt, kmajor=(False, True), axis=1)
+            dx = dx.view(ctx.shape)
+        if any(ctx.needs_input_grad[1:]):
+            dws = [torch.empty_like(w) for w in weights]
+            gemm(grads, [flat], dws, nt, k, m, kmajor=(True, True), axis=3)
+        return (dx, *dws)
 
 
 def shared_input_projections(x, weights, *, optimized=False):
-    """[X W_i^T for W_i in weights]; the fused backward needs 16-bit contiguous operands with every
-    dimension a multiple of 8, otherwise each projection is an ordinary ``linear``."""
-    ok = x.dtype in (torch.bfloat16, torch.float16) and x.is_contiguous() and x.shape[-1] % 8 == 0 and \
-        (x.numel() // x.shape[-1]) % 8 == 0 and \
-        all(w.dtype == x.dtype and w.is_contiguous() and w.ndim == 2 and w.shape[1] == x.shape[-1] and
-            w.shape[0] % 8 == 0 for w in weights)
-    if not ok:
-        return [linear(x, w, optimized=optimized) for w in weights]
-    return list(_SharedInputProjections.apply(x, *weights))
-
+    """[X W_i^T for W_i in weights] for up to three weights; 16-bit contiguous operands whose feature counts
+    are multiples of 8 share their launches, otherwise each projection is an ordinary ``linear``."""
+    if len(weights) <= 3 and x.is_contiguous() and x.numel() and \
+            gemm_ok(x.view(-1, x.shape[-1]), *weights) and \
+            all(w.is_contiguous() and w.ndim == 2 and w.shape[1] == x.shape[-1] and w.shape[0] % 8 == 0 for w in weights):
+        return list(_SharedInputProjections.apply(x, *weights))
+    return [linear(x, w, optimized=optimized) for w in weights]

@@ -1,0 +1,150 @@
+"""q3_gemm: ragged sizes, K-major operands, pieces and K splits against fp64 products, and the fused
+epilogues bit for bit against the plain product followed by the separate kernel."""
+import pytest
+import torch
+
+from _util import max_rel, randn, seeded
+
+from qwen3_triton import _hip as H
+from qwen3_triton.kernels import _ops
+from qwen3_triton.kernels.linear import gemm
+
+pytestmark = pytest.mark.gpu
+# one rounding of the fp32 sum to the storage type: half an ulp of the largest value, 2^-9 (bf16) / 2^-12 (fp16)
+TOL = {torch.bfloat16: 4e-3, torch.float16: 5e-4}
+
+
+def guarded(m, n, dtype):
+    """An [m, n] output inside a larger buffer of sevens: what lies outside must stay."""
+    buf = torch.full((m + 3, n + 16), 7.0, device="cuda", dtype=dtype)
+    return buf, buf[:m, :n]
+
+
+def untouched(buf, m, n):
+    return bool((buf[m:] == 7).all()) and bool((buf[:, n:] == 7).all())
+
+
+# edges of the 32 / 64 / 128 / 256 tiles and of the 64-wide k-tile, single rows, long k (splits), many tiles
+SHAPES = [(1, 8, 8), (17, 64, 72), (33, 136, 64), (65, 4096, 4096), (128, 1024, 1032), (257, 264, 200),
+          (333, 4096, 1024), (2050, 4104, 328), (40, 512, 12288)]
+
+
+@pytest.mark.parametrize("m,n,k", SHAPES)
+@pytest.mark.parametrize("layout", ["NT", "NN", "TN"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_layouts(m, n, k, layout, dtype):
+    if layout == "TN":   # the weight gradient's shape: features x features over a ragged token count
+        m, k = -(-k // 8) * 8, m
+    print(f"q3_gemm {layout} {m}x{n}x{k} {dtype}", flush=True)
+    gen = seeded(m + 3 * n + k)
+    a, b = randn(m, k, gen=gen, dtype=dtype).cuda(), randn(n, k, gen=gen, dtype=dtype).cuda()
+    buf, c = guarded(m, n, dtype)
+    ao = a.t().contiguous() if layout == "TN" else a
+    bo = b if layout == "NT" else b.t().contiguous()
+    gemm([ao], [bo], [c], m, n, k, kmajor=(layout == "TN", layout != "NT"))
+    assert max_rel(c, a.double() @ b.double().t()) < TOL[dtype]
+    assert untouched(buf, m, n)
+
+
+def test_operands_in_place():
+    """Row-strided operands (column blocks of wider matrices) and NaN / infinity around them: nothing outside
+    the operand enters a product."""
+    gen = seeded(3)
+    m, n, k = 70, 40, 88
+    for kmajor in ((False, False), (False, True), (True, True)):
+        mm = 72 if kmajor[0] else m
+        a = torch.full((200, 160), float("nan")).bfloat16()
+        b = torch.full((200, 160), float("inf")).bfloat16()
+        ra, rb = (k, mm) if kmajor[0] else (mm, k), (k, n) if kmajor[1] else (n, k)
+        a[:ra[0], 8:8 + ra[1]] = randn(*ra, gen=gen, dtype=torch.bfloat16)
+        b[:rb[0], 16:16 + rb[1]] = randn(*rb, gen=gen, dtype=torch.bfloat16)
+        av, bv = a.cuda()[:ra[0], 8:8 + ra[1]], b.cuda()[:rb[0], 16:16 + rb[1]]
+        c = torch.empty(mm, n, device="cuda", dtype=torch.bfloat16)
+        gemm([av], [bv], [c], mm, n, k, kmajor=kmajor)
+        e = (av.double().t() if kmajor[0] else av.double()) @ (bv.double() if kmajor[1] else bv.double().t())
+        assert max_rel(c, e) < TOL[torch.bfloat16], kmajor
+
+
+@pytest.mark.parametrize("m,ns,k", [(65, (4096, 1024, 1024), 4096), (333, (256, 64, 72), 512), (9, (40, 8), 104)])
+def test_pieces(m, ns, k):
+    """q/k/v-style pieces along n, k and m against fp64."""
+    gen = seeded(sum(ns) + m)
+    dt = torch.bfloat16
+    x = randn(m, k, gen=gen, dtype=dt).cuda()
+    ws = [randn(n, k, gen=gen, dtype=dt).cuda() for n in ns]
+    dys = [randn(m, n, gen=gen, dtype=dt).cuda() for n in ns]
+    bufs = [guarded(m, n, dt) for n in ns]
+    print(f"q3_gemm pieces {m} {ns} {k}", flush=True)
+    gemm([x], ws, [c for _, c in bufs], m, sum(ns), k, axis=2)
+    for (buf, c), w, n in zip(bufs, ws, ns):
+        assert max_rel(c, x.double() @ w.double().t()) < TOL[dt] and untouched(buf, m, n)
+    dx = torch.empty(m, k, device="cuda", dtype=dt)
+    gemm(dys, ws, [dx], m, k, sum(ns), kmajor=(False, True), axis=1)
+    assert max_rel(dx, sum(d.double() @ w.double() for d, w in zip(dys, ws))) < TOL[dt]
+    bufs = [guarded(n, k, dt) for n in ns]
+    gemm(dys, [x], [c for _, c in bufs], sum(ns), k, m, kmajor=(True, True), axis=3)
+    for (buf, c), d, n in zip(bufs, dys, ns):
+        assert max_rel(c, d.double().t() @ x.double()) < TOL[dt] and untouched(buf, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(65, 4096, 4096), (20, 264, 4096), (333, 4096, 1024), (600, 256, 64), (3, 8, 8)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_epilogues(m, n, k, dtype):
+    """Residual (in place too), residual + norm, gate/up and the SwiGLU backward: bit-equal to the plain product
+    followed by the add / norm / SwiGLU kernels (the fused norm sums its squares in another order)."""
+    print(f"q3_gemm epilogues {m}x{n}x{k} {dtype}", flush=True)
+    gen = seeded(m + n + 5 * k)
+    x = randn(m, k, gen=gen, dtype=dtype).cuda()
+    w, w2 = (randn(n, k, gen=gen, dtype=dtype, scale=0.05).cuda() for _ in range(2))
+    res, nw = randn(m, n, gen=gen, dtype=dtype).cuda(), randn(n, gen=gen, dtype=dtype).cuda()
+    y = torch.empty(m, n, device="cuda", dtype=dtype)
+    gemm([x], [w], [y], m, n, k)
+    e = _ops.add(res, y)
+    out = torch.empty_like(y)
+    gemm([x], [w], [out], m, n, k, epilogue=H.GEMM_RESIDUAL, res=res)
+    assert torch.equal(out, e)
+    c, h = res.clone(), torch.empty_like(y)
+    gemm([x], [w], [c], m, n, k, epilogue=H.GEMM_RESIDUAL_NORM, res=c, norm=(nw, 1e-6, h))
+    eh = _ops.rmsnorm_fwd(e, nw, 1e-6)
+    assert torch.equal(c, e)
+    # 1 / rms may differ in its last fp32 bit: a few values one rounding step (2^-8 / 2^-11 of the value) apart
+    assert (h != eh).float().mean().item() < 0.01 and max_rel(h, eh) <= (8e-3 if dtype == torch.bfloat16 else 1e-3)
+    g, u, sy, sy2 = (torch.empty_like(y) for _ in range(4))
+    gemm([x], [w, w2], [sy], m, n, k, epilogue=H.GEMM_GATE_UP, g=g, u=u)
+    assert torch.equal(sy, _ops.swiglu_fwd(g, u))
+    assert max_rel(g, x.double() @ w.double().t()) < TOL[dtype] and max_rel(u, x.double() @ w2.double().t()) < TOL[dtype]
+    gemm([x], [w, w2], [sy2], m, n, k, epilogue=H.GEMM_GATE_UP)
+    assert torch.equal(sy2, sy)
+    wk = w.t().contiguous()   # [k, n]: K-major
+    dy, dg, du = (torch.empty_like(y) for _ in range(3))
+    gemm([x], [wk], [dg, du], m, n, k, kmajor=(False, True), epilogue=H.GEMM_SWIGLU_BWD, g=g, u=u)
+    eg, eu = _ops.swiglu_bwd(g, u, (x.double() @ w.double().t()).to(dtype))
+    assert max_rel(dg, eg) <= 4 * TOL[dtype] and max_rel(du, eu) <= 4 * TOL[dtype]   # dY rounds from fp32 and from fp64
+    if k < 1024:   # unsplit plain product: the same fp32 sums
+        gemm([x], [wk], [dy], m, n, k, kmajor=(False, True))
+        eg, eu = _ops.swiglu_bwd(g, u, dy)
+        assert torch.equal(dg, eg) and torch.equal(du, eu)
+
+
+def test_refusals():
+    x = torch.zeros(16, 64, device="cuda", dtype=torch.bfloat16)
+    c = torch.zeros(16, 16, device="cuda", dtype=torch.bfloat16)
+    for a, b, kw in ((x[:, 4:60], x[:, 4:60], {}),                     # 8-byte aligned rows
+                     (x, x, dict(kmajor=(True, False))),               # K-major A with a k-contiguous B
+                     (x, x, dict(epilogue=H.GEMM_RESIDUAL_NORM)),      # no residual, norm weight or output
+                     (x, x, dict(epilogue=H.GEMM_GATE_UP))):           # one weight only
+        with pytest.raises(RuntimeError):
+            gemm([a], [b], [c], 16, 16, a.shape[1], **kw)
+    big = torch.zeros(65, 4096, device="cuda", dtype=torch.bfloat16)
+    d = H.GemmDesc()
+    d.dtype, d.pieces, d.m, d.n, d.k = H.BF16, 1, 65, 65, 4096
+    for f in ("a", "b"):
+        getattr(d, f)[0], getattr(d, "ld" + f)[0] = big.data_ptr(), 4096
+    out = torch.zeros(65, 72, device="cuda", dtype=torch.bfloat16)
+    d.c[0], d.ldc[0], d.n = out.data_ptr(), 72, 64
+    import ctypes
+    need = H.query("q3_gemm_workspace_bytes", ctypes.addressof(d))
+    assert need > 0
+    ws = torch.empty(need, device="cuda", dtype=torch.uint8)
+    with pytest.raises(RuntimeError):   # a workspace below the stated size is refused before any launch
+        H.call("q3_gemm", ctypes.addressof(d), ws.data_ptr(), need - 16, H.stream())
