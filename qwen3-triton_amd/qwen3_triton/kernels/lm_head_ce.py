@@ -7,14 +7,14 @@ columns: each chunk's fp32 logits come from the matrix-core GEMM (h . W_c^T) int
 final merge gives lse and the token-mean loss.  On the matrix-core path the logits GEMM's epilogue also
 keeps each chunk's logits in the activation dtype (bf16: the reference's own lm_head output, whose
 [T, V] copy it materialises too), and the statistics are formed from those stored values; the backward
-turns them in place into dz = (softmax - onehot) * up / count plus dz^T, writes dW_c = dz_c^T . h per
-chunk and dX = dz . W in one GEMM.  Other shapes recompute each chunk's logits in the backward.  The
-same math as ``linear`` followed by ``causal_cross_entropy``.
+turns them in place into dz = (softmax - onehot) * up / count and forms dW = dz^T . h and dX = dz . W from
+them as they lie, one GEMM each, for any token count.  Other shapes recompute each chunk's logits in the
+backward.  The same math as ``linear`` followed by ``causal_cross_entropy``.
 """
 import torch
 
 from . import _ops
-from .linear import gemm_nt_into, matmul_into
+from .linear import gemm, gemm_nt_into, gemm_ok, matmul_into
 
 DEFAULT_CHUNK = 16384
 
@@ -52,13 +52,12 @@ class _LMHeadCE(torch.autograd.Function):
         z = None
         if _mfma_ok(hidden, weight) and h % 64 == 0:
             # logits GEMM with the statistics epilogue: one partial per 128 logit columns, no fp32
-            # logits in memory.  Where the shapes allow, the epilogue also keeps the logits in the
-            # activation dtype (the reference's bf16 lm_head output) for the backward, which then
-            # needs no second logits GEMM.
+            # logits in memory.  The epilogue also keeps the logits in the activation dtype (the
+            # reference's bf16 lm_head output) for the backward, which then needs no second logits GEMM.
             groups = [-(-min(chunk, v - c * chunk) // 128) for c in range(nch)]
             st = _ops.CEState(b * s, sum(groups), hidden.device)
-            if (b * s) % 8 == 0 and chunk % 8 == 0:
-                z = torch.empty((b * s, -(-v // 64) * 64), device=hidden.device, dtype=hidden.dtype)
+            if chunk % 8 == 0 and gemm_ok(x, weight):
+                z = torch.empty((b * s, v), device=hidden.device, dtype=hidden.dtype)
             part0 = 0
             for c in range(nch):
                 c0 = c * chunk
@@ -92,22 +91,16 @@ class _LMHeadCE(torch.autograd.Function):
         mfma = _mfma_ok(x, weight) and t % 8 == 0
         z, ctx.z = ctx.z, None   # consumed: dz overwrites the stored logits in place
         if z is not None:
-            # dz of every chunk from the stored logits, in place, and its transpose (the dW operand);
-            # dW_c = dz_c^T . x per chunk, dX = dz . W in one GEMM over the whole vocabulary.
-            vp = z.shape[1]
-            if vp > v:
-                z[:, v:].zero_()
-            wt = _ops.transpose_last2(weight, pad_to=64)  # [H, Vp]
-            xt = _ops.transpose_last2(x)                  # [H, T]
-            dzt = torch.empty((chunk, t), device=x.device, dtype=x.dtype)
-            for c in range(-(-v // chunk)):
-                c0 = c * chunk
-                n = min(chunk, v - c0)
-                _ops.ce_grad_t(z[:, c0:], n, c0, tgt, lse, count, up, z[:, c0:], dzt, v, ctx.ignore)
-                gemm_nt_into(dzt, t, xt, t, dw[c0:c0 + n], n, h, t)
-            dx = torch.empty((t, h), device=x.device, dtype=x.dtype)
-            gemm_nt_into(z, vp, wt, vp, dx, t, h, vp)
-            return dx.view(b, s, h), dw, None, None, None
+            # dz from the stored logits, in place; dW = dz^T . x and dX = dz . W read it as it lies
+            _ops.ce_grad(z, v, v, 0, tgt, lse, count, up, z, v, v, ctx.ignore)
+            dx = None
+            if ctx.needs_input_grad[1]:
+                gemm([z], [x], [dw], v, h, t, kmajor=(True, True))
+            if ctx.needs_input_grad[0]:
+                dx = torch.empty((t, h), device=x.device, dtype=x.dtype)
+                gemm([z], [weight], [dx], t, h, v, kmajor=(False, True))
+                dx = dx.view(b, s, h)
+            return dx, dw, None, None, None
         if mfma and h % 64 == 0:
             # Every chunk's dz lands in one [T, Vp] buffer (Vp = V rounded up to 64, zero pad) written
             # by the logits GEMM's CE-gradient epilogue; dW_c = dz_c^T . x per chunk, and dX = dz . W
