@@ -82,6 +82,10 @@ struct Args {
   u16 *g, *u;
   const u16 *gin, *uin;
   int64_t ldgu;
+  // cross-entropy statistics (c[0] takes the logits): target columns, partials [group][ldp]
+  const int64_t* tgt;
+  float *m_part, *s_part, *pick;
+  int64_t part0, ldp, col0;
 };
 
 // Work item -> (tile, split): each XCD (workgroup ids congruent mod 8) takes a contiguous range of items,
@@ -100,7 +104,9 @@ Q3_DEV void work_coords(int bid, int tiles_m, int tiles_n, int splits, int& tm, 
   tn = (w % width) / gsize;
 }
 
-// EPI 0: plain / residual / split partials; 3: gate/up SwiGLU; 5: SwiGLU backward.  KP: A and B in pieces along K.
+// EPI 0: plain / residual / split partials; 2: cross-entropy statistics (per row and 128-column group: the max and the
+// sum of exp(z - max) to m_part / s_part [part0 + group][row], the logit of column tgt[row] - col0 to pick[row]) of
+// the rounded logits, which are stored too; 3: gate/up SwiGLU; 5: SwiGLU backward.  KP: A and B in pieces along K.
 template <typename T, int BM, int BN, int WM, int WN, int STAGES, bool AT, bool BT, int EPI, bool KP>
 __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
   constexpr int NW = WM * WN;
@@ -400,7 +406,57 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
       const int c = lane % CH;
       const int rlim = mrows - ma - wm * TMW;  // valid rows / columns of the wave's block
       auto row_chunk = [&](int r) { return *reinterpret_cast<const i32x4*>(wl + r * (NC * 2) + ((c ^ swz(r)) << 4)); };
-      if constexpr (EPI == 3) {
+      if constexpr (EPI == 2) {
+        // The logits are rounded into the staged block first, so their accumulators are dead before the statistics'
+        // temporaries are live; then each row's 16 chunks (16 lanes) are read once, for the store and the statistics.
+        static_assert(TNW == 128 && CH == 16, "one statistics partial per wave and row");
+        const int clim = ncols - nb - wn * TNW;
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+          for (int j = 0; j < FN; ++j)
+            stage_out(i, j, pack2<T>(acc[i][j][0], acc[i][j][1]), pack2<T>(acc[i][j][2], acc[i][j][3]));
+        lds_wait();
+        __builtin_amdgcn_wave_barrier();
+        const int64_t part = (ar.part0 + (nb + wn * TNW) / 128) * ar.ldp;
+        const int have = min(clim - c * 8, 8);  // columns of this lane's chunk
+#pragma unroll 2
+        for (int q = 0; q < TMW / RPI; ++q) {
+          const int r = q * RPI + lane / CH;
+          const int row = ma + wm * TMW + r;
+          const i32x4 raw = row_chunk(r);
+          Vec<T> v = unpack_vec<T>(raw);
+          int64_t t = -1;
+          if (r < rlim) {
+            t = ar.tgt[row] - ar.col0 - (nb + wn * TNW + c * 8);  // target within the lane's chunk
+            u16* dst = C + (int64_t)row * ldc + nb + wn * TNW + c * 8;
+            if (have == 8) {
+              *reinterpret_cast<i32x4*>(dst) = raw;
+            } else {
+#pragma unroll
+              for (int e = 0; e < 8; ++e)
+                if (e < have) dst[e] = (u16)((uint32_t)raw[e >> 1] >> (16 * (e & 1)));
+            }
+          }
+          float mx = -INFINITY;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            if (e >= have) v.v[e] = -INFINITY;
+            mx = fmaxf(mx, v.v[e]);
+            if (e == t && e < have) ar.pick[row] = v.v[e];
+          }
+          mx = group_max<16>(mx);
+          float sm = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) sm += mx == -INFINITY ? 0.f : __expf(v.v[e] - mx);
+          sm = group_sum<16>(sm);
+          if (c == 0 && r < rlim && clim > 0) {  // a wave past the last column has no partial
+            ar.m_part[part + row] = mx;
+            ar.s_part[part + row] = sm;
+          }
+        }
+        return;
+      } else if constexpr (EPI == 3) {
         const int64_t o0 = (int64_t)(ma + wm * TMW) * ldc + (nb + wn * TNW) / 2 + c * 8;
         const int clim = (ncols - nb - wn * TNW) / 2;
         // G and U rounded and packed first: half the registers, and every output forms from the rounded values

@@ -330,4 +330,38 @@ int q3_gemm(const q3_gemm_desc* d, void* workspace, size_t workspace_bytes, hipS
   return q3_rmsnorm_fwd(d->dtype, d->c[0], d->norm_w, d->y, d->m, d->n, d->eps, stream);
 }
 
+// LM-head logits A B^T, stored, with their cross-entropy statistics (q3hip.h): 256 x 256 tiles, 128 x 256 when
+// those would leave half of the last (or only) row of tiles empty.
+int q3_gemm_nt_ce_stats_store(int dtype, const void* A, int64_t lda, const void* B, int64_t ldb, int64_t M, int64_t N,
+                              int64_t K, int64_t col0, const int64_t* tgt, float* m_part, float* s_part, float* pick,
+                              int64_t part0, int64_t ldp, void* z, int64_t ldz, hipStream_t stream) {
+  Q3_REQUIRE((dtype == Q3_BF16 || dtype == Q3_F16) && tgt && m_part && s_part && pick);
+  Q3_REQUIRE(M > 0 && N > 0 && K > 0 && M < (1ll << 31) - 256 && N < (1ll << 30) && K < (1ll << 31) && K % 64 == 0);
+  Q3_REQUIRE(operand_ok(A, lda, M, K, false) && operand_ok(B, ldb, N, K, false) && ldp >= M && part0 >= 0);
+  Q3_REQUIRE(z && ldz >= N && ldz % 8 == 0 && al16(z));
+  Args a{};
+  a.a.p[0] = (const u16*)A;
+  a.a.ld[0] = lda;
+  a.b.p[0] = (const u16*)B;
+  a.b.ld[0] = ldb;
+  a.M = M;
+  a.N = N;
+  a.K = K;
+  a.pieces = a.splits = 1;
+  a.c[0] = z;
+  a.ldc[0] = ldz;
+  a.tgt = tgt;
+  a.m_part = m_part;
+  a.s_part = s_part;
+  a.pick = pick;
+  a.part0 = part0;
+  a.ldp = ldp;
+  a.col0 = col0;
+  const bool big = M > 128 && (M % 256 == 0 || M % 256 > 128 || M > 2048);
+  a.tms = (int)cdiv(M, big ? 256 : 128);
+  a.tns = (int)cdiv(N, 256);
+  Q3_REQUIRE((int64_t)a.tms * a.tns < (1ll << 31));
+  return q3gemm::launch_tile_nt(dtype, big ? 0 : 1, 2, a, stream);
+}
+
 }  // extern "C"

@@ -148,3 +148,29 @@ def test_refusals():
     ws = torch.empty(need, device="cuda", dtype=torch.uint8)
     with pytest.raises(RuntimeError):   # a workspace below the stated size is refused before any launch
         H.call("q3_gemm", ctypes.addressof(d), ws.data_ptr(), need - 16, H.stream())
+
+
+@pytest.mark.parametrize("b,s,h,v", [(1, 2, 64, 8), (1, 129, 64, 264), (3, 67, 128, 1000), (1, 257, 64, 520)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_lm_head_ragged(b, s, h, v, dtype):
+    """The fused LM head + loss at token counts off the tile grid: loss and gradients against fp64, a second
+    backward through the same graph equal to the first."""
+    from qwen3_triton.kernels.lm_head_ce import lm_head_cross_entropy
+    print(f"lm_head {b}x{s} {h} -> {v} {dtype}", flush=True)
+    gen = seeded(b * s + v)
+    x0, w0 = randn(b, s, h, gen=gen, dtype=dtype), randn(v, h, gen=gen, dtype=dtype, scale=0.1)
+    labels = torch.randint(0, v, (b, s), generator=gen)
+    labels[0, s // 2:s // 2 + s // 8] = -100
+    x, w = x0.cuda().requires_grad_(), w0.cuda().requires_grad_()
+    loss = lm_head_cross_entropy(x, w, labels.cuda())
+    first = torch.autograd.grad(loss, [x, w], retain_graph=True)
+    second = torch.autograd.grad(loss, [x, w])
+    xr, wr = x0.double().requires_grad_(), w0.double().requires_grad_()
+    z = xr @ wr.t()
+    e = torch.nn.functional.cross_entropy(z[:, :-1].reshape(-1, v), labels[:, 1:].reshape(-1), ignore_index=-100)
+    grads = torch.autograd.grad(e, [xr, wr])
+    assert abs(float(loss.detach()) - float(e)) <= 1e-3 * abs(float(e))
+    # logits and dz each round once to the storage type (2^-9 / 2^-12 of values up to a few times the rms)
+    for a, c, g in zip(first, second, grads):
+        assert torch.equal(a, c)
+        assert max_rel(a, g) <= (2e-2 if dtype == torch.bfloat16 else 3e-3)
