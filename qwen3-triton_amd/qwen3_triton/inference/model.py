@@ -191,14 +191,23 @@ class TritonQwen3Inference(nn.Module):
         cache.admit(self._cache_owner, b, s)
         if type(logits_to_keep) is not int or not 0 <= logits_to_keep <= s:
             raise ValueError('logits_to_keep must be 0 or within current sequence length')
-        if validate_ids and not bool(((input_ids >= 0) & (input_ids < self.config.vocab_size)).all()):
-            raise ValueError('Token ID outside vocabulary')
         start = cache.length
         if start_dev is not None and s != 1:
             raise ValueError('device-resident positions are for single-token decode steps')
+        x = None
+        if validate_ids:
+            # the embedding kernel's own range flag is the check: one launch and one synchronisation; the
+            # cache is untouched when it fails
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError('token IDs cannot be validated during graph capture')
+            try:
+                x = embedding(input_ids, self.model.embed_tokens.weight)
+            except ValueError:
+                raise ValueError('Token ID outside vocabulary') from None
         pos = kernels.positions(b, s, start, self.device, start_dev)
         try:
-            x = embedding(input_ids, self.model.embed_tokens.weight)
+            if x is None:
+                x = embedding(input_ids, self.model.embed_tokens.weight)
             cos, sin = self.model.rotary_emb(pos, torch.bfloat16)
             fused = self.gemv and kernels.decode_linear_ok(x, self.lm_head.weight)
             layers = self.model.layers
