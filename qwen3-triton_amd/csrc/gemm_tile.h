@@ -514,7 +514,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
         lds_wait();
         __builtin_amdgcn_wave_barrier();
         // batches of up to 4 row passes: the batch's residual (or g / u) rows are all in flight before their use
-        constexpr int NP = TMW / RPI, BP = NP < 4 ? NP : 4;
+        constexpr int NP = TMW / RPI, BP = NP % 4 == 0 ? 4 : NP % 3 == 0 ? 3 : NP < 4 ? NP : 1;
         static_assert(NP % BP == 0, "row passes");
 #pragma unroll
         for (int q0 = 0; q0 < NP; q0 += BP) {

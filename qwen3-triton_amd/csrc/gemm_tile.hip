@@ -23,8 +23,13 @@ struct Cfg {
   int bm, bn, conc;
   double solo, full;
 };
-constexpr Cfg kCfg[6] = {{256, 256, 1, 1.27, 1.48}, {128, 256, 1, 0.86, 0.94}, {128, 128, 1, 0.48, 0.62},
-                         {64, 128, 1, 0.28, 0.32},  {64, 64, 2, 0.34, 0.70},   {32, 64, 3, 0.27, 1.04}};
+constexpr int kNumCfg = 8;
+constexpr Cfg kCfg[kNumCfg] = {{256, 256, 1, 1.27, 1.48}, {128, 256, 1, 0.86, 0.94}, {128, 128, 1, 0.48, 0.62},
+                               {64, 128, 1, 0.28, 0.32},  {64, 64, 2, 0.34, 0.70},   {32, 64, 3, 0.27, 1.04},
+                               {192, 256, 1, 0.98, 1.25}, {192, 128, 1, 0.61, 0.68}};
+// Instantiated layouts: the 192-row tiles for a k-contiguous A (they fill the CUs where 256 rows would leave the
+// last row of tiles half empty: 1500 x 24576 x 4096 247 against 279 us), 32 rows for two k-contiguous operands.
+bool cfg_for(int c, bool at, bool bt) { return c < 5 || (c == 5 ? !bt : !at); }
 constexpr int kSplits[6] = {1, 2, 3, 4, 6, 8};
 constexpr int64_t kMinSplitK = 512;  // k per split
 
@@ -66,21 +71,22 @@ int64_t tile_cols(const Args& a, int bn) {
 // combine: what the combining pass adds besides its traffic (us): a launch (4.5 measured on small products), or
 // next to nothing where the pass also forms the norm that an unsplit product would leave to a launch of its own.
 // can_split: the product may be formed as partial products (plain or residual epilogue, 16-byte columns).
-Plan plan_for(const Args& a, bool kmajor, bool can_split, double combine, int64_t row0 = 0) {
+Plan plan_for(const Args& a, bool at, bool bt, bool can_split, double combine, int64_t row0 = 0) {
   Plan best{0, 1};
-  double bt = 0.0;
+  double best_t = 0.0;
   const int64_t rows = a.M - row0;
-  for (int c = 0; c < (kmajor ? 5 : 6); ++c) {
-    if (kCfg[c].bm >= 2 * rows && c < (kmajor ? 4 : 5)) continue;  // more than half of the tile's rows empty
+  for (int c = 0; c < kNumCfg; ++c) {
+    if (!cfg_for(c, at, bt)) continue;
+    if (kCfg[c].bm >= 2 * rows && kCfg[c].bm > (bt ? 64 : 32)) continue;  // more than half of the tile's rows empty
     const int64_t tiles = (tile_rows(a, kCfg[c].bm) - row0 / kCfg[c].bm) * tile_cols(a, kCfg[c].bn);
     for (int sp : kSplits) {
       // a grid that fills the chip by itself is not split: its partial products would outgrow the caches
       // (6144 x 4096 x 8192 in two splits: 390 + 43 us against 300 us in two launches, below)
       if (sp > 1 && (!can_split || a.K / sp < kMinSplitK || tiles >= 256 * kCfg[c].conc)) break;
       const double t = estimate(c, sp, tiles, rows, a.N, a.K, combine);
-      if (bt == 0.0 || t < bt) {
+      if (best_t == 0.0 || t < best_t) {
         best = {c, sp};
-        bt = t;
+        best_t = t;
       }
     }
   }
@@ -291,14 +297,14 @@ extern "C" {
 size_t q3_gemm_workspace_bytes(const q3_gemm_desc* d) {
   Call c;
   if (!parse(d, c)) return 0;
-  const Plan p = plan_for(c.a, c.bt, c.can_split, c.combine);
+  const Plan p = plan_for(c.a, c.at, c.bt, c.can_split, c.combine);
   return p.splits > 1 ? (size_t)p.splits * (size_t)c.a.M * (size_t)c.a.N * sizeof(float) : 0;
 }
 
 int q3_gemm(const q3_gemm_desc* d, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   Call c;
   Q3_REQUIRE(parse(d, c));
-  Plan p = plan_for(c.a, c.bt, c.can_split, c.combine);
+  Plan p = plan_for(c.a, c.at, c.bt, c.can_split, c.combine);
   const bool norm = d->epilogue == Q3_GEMM_RESIDUAL_NORM;
   if (p.splits > 1) {
     Q3_REQUIRE(workspace && al16(workspace) &&
@@ -323,7 +329,7 @@ int q3_gemm(const q3_gemm_desc* d, void* workspace, size_t workspace_bytes, hipS
   if (m1 > 0) {
     const int rc = launch(c, p, 0, m1, d->dtype, stream);
     if (rc != 0) return rc;
-    p = plan_for(c.a, c.bt, false, c.combine, m1);
+    p = plan_for(c.a, c.at, c.bt, false, c.combine, m1);
   }
   const int rc = launch(c, p, m1, c.a.M, d->dtype, stream);
   if (rc != 0 || !norm) return rc;

@@ -10,6 +10,8 @@ template <typename T, int EPI> static int nt(int cfg, const Args& a, hipStream_t
     case 2: return launch_tile<T, 128, 128, 2, 2, 3, false, false, EPI>(a, s);
     case 3: return launch_tile<T, 64, 128, 2, 4, 4, false, false, EPI>(a, s);
     case 4: return launch_tile<T, 64, 64, 2, 2, 4, false, false, EPI>(a, s);
+    case 6: return launch_tile<T, 192, 256, 4, 2, 2, false, false, EPI>(a, s);
+    case 7: return launch_tile<T, 192, 128, 4, 2, 3, false, false, EPI>(a, s);
     default: return launch_tile<T, 32, 64, 2, 2, 4, false, false, EPI>(a, s);
   }
 }
