@@ -34,10 +34,13 @@ static_assert(4 * kRed <= 4 * kWaveLds, "the fold reuses the rings");
 Q3_DEV i32x4 ld16(const u16* p) { return *reinterpret_cast<const i32x4*>(p); }
 Q3_DEV bf16x8_t as_frag(i32x4 v) { return __builtin_bit_cast(bf16x8_t, v); }
 // 8 bytes by the gfx950 transpose read: within each 16-lane group, lane j receives element j % 4 of
-// the 8-byte pieces addressed by lanes j / 4 + 4 k, k = 0..3.
-Q3_DEV i32x2 ldtr(const char* p) {
-  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t*)p));
+// the 8-byte pieces addressed by lanes j / 4 + 4 k, k = 0..3.  Read through a __restrict parameter: without alias
+// information the compiler waits for every direct-to-LDS load in flight before such a read.
+typedef __attribute__((address_space(3))) v4s_t* lds_v4s;
+Q3_DEV i32x2 ldtr_at(lds_v4s __restrict p) {
+  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p));
 }
+Q3_DEV i32x2 ldtr(const char* p) { return ldtr_at((lds_v4s)p); }
 // 16-byte chunk swizzle of the 256-byte query rows: conflict-free row reads (16 rows of one chunk
 // column) and distinct 32-byte bank groups for the 8 rows of each half-wave transpose read.
 Q3_DEV int qswz(int r) { return 2 * ((r & 3) | (((r >> 3) & 1) << 2)) + ((r >> 4) & 1); }
@@ -131,28 +134,55 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     const int nq = qstart < Lq ? (Lq - qstart + kBM - 1) / kBM : 0;
     const int total = hpw * nq;
 
-    auto issue = [&](int u) {  // 8 + 8 wave loads of 4 rows x 256 B (Q, dO), one of lse / delta
-      const int hh = u / nq, q0 = qstart + (u % nq) * kBM;
-      const int h = hk * ratio + wave + 4 * hh;
-      const int64_t bh = (int64_t)b * Hq + h;
-      // wave-uniform bases (SGPRs) + 32-bit per-lane byte offsets
-      const char* Qb = reinterpret_cast<const char*>(Q + b * qsb + h * qsh);
-      const char* dOb = reinterpret_cast<const char*>(dO + b * qsb + h * qsh);
-      char* base = wl + (u % kST) * kStage;
+    // Tile loads: 8 + 8 wave loads of 4 rows x 256 B (Q, dO), one of lse / delta, through range-checked buffer
+    // descriptors that advance by a tile: rows past the end read zeros, and a load is one instruction beside its
+    // LDS address (addresses formed per load, with a clamped row: 125 instructions a tile, about 700 of the 4100
+    // cycles a wave spent on one).
+    uint32_t voff[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int r = 4 * i + (lane >> 4);
+      voff[i] = (uint32_t)((r * qss + (((lane & 15) ^ qswz(r)) * 8)) * 2);
+    }
+    const u16 *qp = nullptr, *dop = nullptr;  // the next tile to load
+    int qrem = 0, iq = 0, ih = 0;             // its 16-byte units to the operand's end; its tile and head
+    const float* side = nullptr;
+    auto head = [&]() {
+      const int h = hk * ratio + wave + 4 * ih;
+      const int64_t base = b * qsb + h * qsh + qstart * qss;
+      qp = Q + base;
+      dop = dO + base;
+      qrem = (int)(((Lq - 1 - qstart) * qss + kD) >> 3);
+      side = (lane < 32 ? LSE : Delta) + ((int64_t)b * Hq + h) * Lq;
+    };
+    auto issue = [&](int stage) {
+      char* base = wl + stage * kStage;
+      const int bytes = min(qrem, 0x7ffffff) * 16;  // tile offsets stay below
+      const auto rq = __builtin_amdgcn_make_buffer_rsrc((void*)qp, 0, bytes, 0x00027000);
+      const auto rd = __builtin_amdgcn_make_buffer_rsrc((void*)dop, 0, bytes, 0x00027000);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const int r = 4 * i + (lane >> 4);
-        const int c = (lane & 15) ^ qswz(r);
-        const uint32_t src = (uint32_t)(min(q0 + r, Lq - 1) * (int)qss + c * 8) * 2u;
-        __builtin_amdgcn_global_load_lds(Qb + src, (lds_vp)(base + i * 1024), 16, 0, 0);
-        __builtin_amdgcn_global_load_lds(dOb + src, (lds_vp)(base + kTB + i * 1024), 16, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rq, (lds_vp)(base + i * 1024), 16, voff[i], 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rd, (lds_vp)(base + kTB + i * 1024), 16, voff[i], 0, 0, 0);
       }
-      const uint32_t qq = (uint32_t)min(q0 + (lane & 31), Lq - 1) * 4u;
-      const char* side = reinterpret_cast<const char*>((lane < 32 ? LSE : Delta) + bh * Lq);
-      __builtin_amdgcn_global_load_lds(side + qq, (lds_vp)(base + 2 * kTB), 4, 0, 0);
+      __builtin_amdgcn_global_load_lds(side + min(qstart + iq * kBM + (lane & 31), Lq - 1), (lds_vp)(base + 2 * kTB), 4,
+                                       0, 0);
+      if (++iq == nq) {
+        iq = 0;
+        ++ih;
+        if (ih < hpw) head();
+      } else {
+        qp += kBM * qss;
+        dop += kBM * qss;
+        qrem -= (int)(kBM * qss >> 3);
+      }
     };
 
-    if (total > 0) issue(0);
+    if (total > 0) {
+      head();
+      issue(0);
+    }
+    int cq = 0;  // query tile of u within its head
 #pragma nounroll
     for (int u = 0; u < total; ++u) {
       // this wave's reads of the stage about to be refilled (tile u - 1) are complete, then the
@@ -160,26 +190,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
       __builtin_amdgcn_s_waitcnt((15) | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
       asm volatile("" ::: "memory");
       if (u + 1 < total) {
-        issue(u + 1);
+        issue((u + 1) & 1);
         wait_vm(17);
       } else {
         wait_vm(0);
       }
       asm volatile("" ::: "memory");
-      const int q0 = qstart + (u % nq) * kBM;
+      const int q0 = qstart + cq * kBM;
+      cq = cq + 1 == nq ? 0 : cq + 1;
       if (min(q0 + kBM - 1, Lq - 1) + off < k0) continue;  // no query of the tile sees these keys
       // Tiles that cross the diagonal or the end of the queries mask P (a uniform branch around the
       // P computation only: two copies of the whole tile body made the register allocator copy the
       // accumulators between them).
       const bool masked = !(k0 + kBN - 1 <= q0 + off && q0 + kBM - 1 < Lq);
       {
-        const char* qb = wl + (u % kST) * kStage;
+        const char* qb = wl + (u & 1) * kStage;
         const char* db = qb + kTB;
-        const float* side = reinterpret_cast<const float*>(qb + 2 * kTB);
-        const f32x4 l0 = *reinterpret_cast<const f32x4*>(side + 8 * G);
-        const f32x4 l1 = *reinterpret_cast<const f32x4*>(side + 8 * G + 4);
-        const f32x4 d0 = *reinterpret_cast<const f32x4*>(side + kBM + 8 * G);
-        const f32x4 d1 = *reinterpret_cast<const f32x4*>(side + kBM + 8 * G + 4);
+        const float* ld = reinterpret_cast<const float*>(qb + 2 * kTB);
+        const f32x4 l0 = *reinterpret_cast<const f32x4*>(ld + 8 * G);
+        const f32x4 l1 = *reinterpret_cast<const f32x4*>(ld + 8 * G + 4);
+        const f32x4 d0 = *reinterpret_cast<const f32x4*>(ld + kBM + 8 * G);
+        const f32x4 d1 = *reinterpret_cast<const f32x4*>(ld + kBM + 8 * G + 4);
 
         // S and dP (dP starts from -delta, its row constant, so the products leave dP - delta);
         // MFMA row r16 of query sub-tile t reads query 8 (r16 / 4) + 4 t + r16 % 4, so lane group G
@@ -191,59 +222,73 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
           nl[0][i] = -l0[i] * kLog2e;
           nl[1][i] = -l1[i] * kLog2e;
         }
-        // Fragment reads run one k-step ahead of their MFMAs, behind scheduling fences (without the
-        // fences the scheduler hoists every LDS read of the tile and runs out of registers).
+        // All row fragments first (64 registers), then key sub-tile by key sub-tile: the products of sub-tile
+        // c + 1 run on the matrix cores beside the exponentials of sub-tile c (one wave per SIMD: nothing else
+        // would overlap them).  Tiles that mask P do the same work in sequence.
         f32x4 s[2][kC], dp[2][kC];
-        i32x4 qa[2][2], da[2][2];
-        auto rows = [&](int ks, int buf) {
-  #pragma unroll
+        i32x4 qa[4][2], da[4][2], pp[kC], dd[kC];
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
           for (int t = 0; t < 2; ++t) {
-            qa[buf][t] = *reinterpret_cast<const i32x4*>(qb + roff[ks] + 4 * t * 256);
-            da[buf][t] = *reinterpret_cast<const i32x4*>(db + roff[ks] + 4 * t * 256);
+            qa[ks][t] = *reinterpret_cast<const i32x4*>(qb + roff[ks] + 4 * t * 256);
+            da[ks][t] = *reinterpret_cast<const i32x4*>(db + roff[ks] + 4 * t * 256);
           }
-        };
-        rows(0, 0);
-  #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          __builtin_amdgcn_sched_barrier(0);
-          if (ks < 3) rows(ks + 1, (ks + 1) & 1);
-          const int cb = ks & 1;
-  #pragma unroll
-          for (int t = 0; t < 2; ++t)
-  #pragma unroll
-            for (int c = 0; c < kC; ++c) {
-              s[t][c] = mfma_16x16x32<T>(as_frag(qa[cb][t]), kf[c][ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[t][c]);
-              dp[t][c] = mfma_16x16x32<T>(as_frag(da[cb][t]), vf[c][ks], ks == 0 ? -(t ? d1 : d0) : dp[t][c]);
+        auto sdp = [&](int c) {
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+              s[t][c] = mfma_16x16x32<T>(as_frag(qa[ks][t]), kf[c][ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[t][c]);
+              dp[t][c] = mfma_16x16x32<T>(as_frag(da[ks][t]), vf[c][ks], ks == 0 ? -(t ? d1 : d0) : dp[t][c]);
             }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        i32x4 pp[kC], dd[kC];
-        auto probs = [&](auto mask_c) {
+        };
+        auto prob = [&](int c, auto mask_c) {
           constexpr bool MASK = decltype(mask_c)::value;
-  #pragma unroll
-          for (int c = 0; c < kC; ++c) {
-            float pv[8], dsv[8];
-  #pragma unroll
-            for (int t = 0; t < 2; ++t)
-  #pragma unroll
-              for (int i = 0; i < 4; ++i) {
-                float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][c][i], scale2, nl[t][i]));
-                if constexpr (MASK) {
-                  const int q = q0 + 8 * G + 4 * t + i;
-                  p = (k0 + 16 * c + r16 <= q + off && q < Lq) ? p : 0.f;
-                }
-                pv[4 * t + i] = p;
-                dsv[4 * t + i] = p * dp[t][c][i];
+          float pv[8], dsv[8];
+#pragma unroll
+          for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][c][i], scale2, nl[t][i]));
+              if constexpr (MASK) {
+                const int q = q0 + 8 * G + 4 * t + i;
+                p = (k0 + 16 * c + r16 <= q + off && q < Lq) ? p : 0.f;
               }
-  #pragma unroll
-            for (int w = 0; w < 4; ++w) {
-              pp[c][w] = (int)pack2<T>(pv[2 * w], pv[2 * w + 1]);
-              dd[c][w] = (int)pack2<T>(dsv[2 * w], dsv[2 * w + 1]);
+              pv[4 * t + i] = p;
+              dsv[4 * t + i] = p * dp[t][c][i];
             }
+#pragma unroll
+          for (int w = 0; w < 4; ++w) {
+            pp[c][w] = (int)pack2<T>(pv[2 * w], pv[2 * w + 1]);
+            dd[c][w] = (int)pack2<T>(dsv[2 * w], dsv[2 * w + 1]);
           }
         };
-        if (masked) probs(std::true_type{});
-        else probs(std::false_type{});
+        if (masked) {
+#pragma unroll
+          for (int c = 0; c < kC; ++c) sdp(c);
+#pragma unroll
+          for (int c = 0; c < kC; ++c) prob(c, std::true_type{});
+        } else {
+          sdp(0);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int c = 0; c < kC; ++c) {
+            if (c + 1 < kC) sdp(c + 1);
+            prob(c, std::false_type{});
+            if (c + 1 < kC) {
+#pragma unroll
+              for (int q = 0; q < 8; ++q) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
+              }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
         i32x4 aq[2], ad[2];
         auto trs = [&](int dt, int buf) {
           const i32x2 q0v = ldtr(qb + tr_addr(0, dt)), q1v = ldtr(qb + tr_addr(1, dt));
