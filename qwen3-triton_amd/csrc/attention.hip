@@ -1654,7 +1654,9 @@ int bwd_mfma(const void* q, Lay ql, const void* k, const void* v, Lay kl, const 
       rc = bwd_dq_v3<T, 2>(q, ql, k, v, kl, kt, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, ldkt, scale, s);
     else rc = bwd_dq_v3<T, 1>(q, ql, k, v, kl, kt, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, ldkt, scale, s);
     if (rc) return rc;
-    if (grp % 4 == 0)  // one query head per wave, 48-key wave tiles (attention_bwd.hip)
+    // one query head per wave, 48-key wave tiles (attention_bwd.hip): its buffer descriptors hold 32-bit tile offsets
+    // and count a head's rows in 32-bit units of 16 bytes; wider operands take the kernel below, as other groups do
+    if (grp % 4 == 0 && ql.s < (1 << 24) && ql.s * Lq < ((int64_t)1 << 34))
       return q3i_attn_bwd_dkdv_v4(T::code, q, ql.b, ql.h, ql.s, k, v, kl.b, kl.h, kl.s, dout, lse, delta, dk, dv, B,
                                   Hq, Hkv, Lq, Lk, scale, s);
     dim3 g2((unsigned)(B * Hkv), (unsigned)((Lk + 127) / 128));

@@ -179,3 +179,23 @@ def test_seq_major_layout(l, d, layout):
     src = p ^ ((((p >> 2) ^ (p >> 3)) & 1) * 12)
     assert torch.equal(y, ref[..., src])
 
+
+
+def test_attention_wide_position_stride():
+    """Positions 2^26 elements apart (heads inside a row, the operands in one buffer): rows 16 and up of a 32-row
+    tile lie past the 2 GiB that the grouped dK/dV kernel's tile loads reach, so these operands take the kernels
+    with 64-bit addresses."""
+    print("attention wide position stride", flush=True)
+    q, k, v, do = make(1, 4, 1, 40, 40, 128, torch.bfloat16, seed=11)
+    buf = torch.empty(40 << 26, dtype=torch.bfloat16, device="cuda")
+
+    def wide(t, at):
+        return buf.as_strided(t.shape, (1 << 26, 128, 1 << 26, 1), at).copy_(t)
+    qd, kd, vd, dod = (wide(t, 1024 * i) for i, t in enumerate((q, k, v, do)))
+    o, lse = _ops.attention_fwd(qd, kd, vd, 128 ** -0.5)
+    grads = _ops.attention_bwd(qd, kd, vd, o, lse, dod, 128 ** -0.5)
+    assert max_rel(o, O.scaled_dot_product_attention_reference(q, k, v)) <= FWD_TOL[torch.bfloat16]
+    e = O.scaled_dot_product_attention_backward_reference(q, k, v, do)
+    for a, x, n in zip(grads, e, "qkv"):
+        assert cosine(a, x) >= 0.999, f"d{n} cosine"
+        assert max_rel(a, x) <= GRAD_TOL[torch.bfloat16], f"d{n} max-rel {max_rel(a, x)}"
