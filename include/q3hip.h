@@ -305,9 +305,10 @@ int q3_gemm_strided(int in_dtype, int out_dtype, const void* A, int64_t sam, int
  * uses KV head h/(Hq/Hkv).  LSE and delta are [B,Hq,Lq] fp32 (natural-log LSE; delta =
  * rowsum(O*dO) is backward scratch).  On the matrix-core path (q3_attention_mfma_supported) the
  * caller also passes sequence-major copies [B,H,D,ld] (ld >= L, ld % 16 == 0, zero pad) made by
- * q3_attention_seq_major: vt of V (forward), qt of Q, kt of K and dot of dO (backward; at head_dim
- * 128 only kt is read -- Q and dO are read transposed in LDS -- and qt / dot may be null), and every
- * row must be 16-byte aligned.  Within every 16-position block of such a row the positions are
+ * q3_attention_seq_major: vt of V (forward), qt of Q, kt of K and dot of dO (backward), and every row
+ * must be 16-byte aligned.  At head_dim 128 the operands are read transposed in LDS: the backward reads
+ * none of the copies, the forward reads vt only where V is not 16-byte aligned or kss is 2^24 or more,
+ * and copies that are not read may be null.  Within every 16-position block of such a row the positions are
  * stored in the order 0-3, 8-11, 4-7, 12-15 (the operand order of the matrix-core kernels).
  * Other dtypes/head sizes run a SIMT path that ignores them.
  * Replaces: kernels/attention.py:20-50 + attention_kernels.py:9-253 (_attention_forward_kernel,

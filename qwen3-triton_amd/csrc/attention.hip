@@ -242,7 +242,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int vg = 0; vg < 4; ++vg) {
         const int d = dt * 32 + 8 * vg + 4 * g;
-        typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
         i32x2 w;
         w[0] = (int)pack2<T>(oacc[dt][4 * vg] * inv, oacc[dt][4 * vg + 1] * inv);
         w[1] = (int)pack2<T>(oacc[dt][4 * vg + 2] * inv, oacc[dt][4 * vg + 3] * inv);
@@ -282,12 +281,27 @@ Q3_DEV float xmax4(float x) {  // max over lanes {l, l^16, l^32, l^48}
 Q3_DEV int kswz3(int r) { return (r & 7) | (((r >> 4) & 1) << 3); }
 Q3_DEV int vswz3(int r) { return (r >> 1) & 7; }
 
-template <typename T, int GH, int NW>
+// One wave load of 16 bytes a lane into LDS, zeros from `bytes` on.  A function of its own, not a template's
+// statement: the host pass drops the stub of a kernel template whose descriptor depends on its parameters.
+Q3_DEV void buffer_to_lds(const u16* p, int bytes, uint32_t off, char* dst) {
+  const auto d = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00027000);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(d, (lds_vp)dst, 16, off, 0, 0, 0);
+}
+
+// VR: V is read as its rows lie and its fragments (P.V contracts over keys) come from transpose reads of the
+// tile; otherwise from the sequence-major copy Vt.  The row tile is 16 slots of 1 KB, slot s holding keys s, s + 16,
+// s + 32, s + 48, at a pitch of 1056 bytes: four consecutive keys sit 32 bytes apart modulo the 256-byte bank span and
+// the next four 128 bytes on, so the half-wave of a transpose read touches every bank once, and every fragment of a
+// lane is one base address plus constants.  Against the copy (a launch that reads and writes V; 32/8 heads): B1 S8192
+// 587 -> 571 us, B4 S2048 156 -> 147, B3 S1000 fp16 48.6 -> 42.3, B1 S333 20.5 -> 12.7; with the tile's addresses formed
+// per load in 64 bits S8192 took 612, behind the copy.
+constexpr int kSlot = 1056, kRowTile = 16 * kSlot;
+template <typename T, int GH, int NW, bool VR>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_v3(
     const u16* __restrict__ Q, Lay ql, const u16* __restrict__ K, Lay kl, const u16* __restrict__ Vt,
     u16* __restrict__ O, float* __restrict__ LSE, int Hq, int Hkv, int Lq, int Lk, int ldvt, float scale2) {
   constexpr int D = 128, BN = 64, QT = 32 * (NW / GH);
-  constexpr int KST = BN * D * 2, VST = D * BN * 2;
+  constexpr int KST = BN * D * 2, VST = VR ? kRowTile : D * BN * 2;
   __shared__ __attribute__((aligned(1024))) char lds[2 * KST + 2 * VST];
   char* const kring = lds;
   char* const vring = lds + 2 * KST;
@@ -302,7 +316,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const int q0 = qt * QT + (wave / GH) * 32;
   const u16* Qb = Q + b * ql.b + h * ql.h;
   const u16* Kb = K + b * kl.b + hk * kl.h;
-  const u16* Vb = Vt + (int64_t)(b * Hkv + hk) * D * ldvt;
+  const u16* Vb = VR ? Vt + b * kl.b + hk * kl.h : Vt + (int64_t)(b * Hkv + hk) * D * ldvt;
 
   bf16x8_t qf[2][4];
 #pragma unroll
@@ -317,9 +331,25 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   const int nfull = min(nbw, max(0, (qfirst_w + 1) / BN));  // blocks fully visible to the wave
   const int qpos[2] = {q0 + r16 + off, q0 + 16 + r16 + off};
 
+  // VR: K and V tiles come through range-checked buffer descriptors (rows past the end read zeros), so a lane's
+  // offsets are loop constants; the host keeps kl.s below 2^24 for them.
+  uint32_t kvo[16 / NW], vvo[16 / NW];
+#pragma unroll
+  for (int i = 0; i < 16 / NW; ++i) {
+    const int w = wave + NW * i, r = 4 * w + (lane >> 4);
+    kvo[i] = (uint32_t)((r * (int)kl.s + ((lane & 15) ^ kswz3(r)) * 8) * 2);
+    vvo[i] = (uint32_t)(((w + 16 * (lane >> 4)) * (int)kl.s + (lane & 15) * 8) * 2);
+  }
+  auto bytes = [&](int j) { return (min(Lk - j * BN, BN) - 1) * ((int)kl.s * 2) + 2 * D; };  // of tile j
   auto issueK = [&](int j) {  // 16 wave loads of 4 rows x 256 B, 2 per wave
     const int k0 = j * BN;
     char* base = kring + (j & 1) * KST;
+    if constexpr (VR) {
+      const int n = bytes(j);
+#pragma unroll
+      for (int i = 0; i < 16 / NW; ++i) buffer_to_lds(Kb + k0 * kl.s, n, kvo[i], base + (wave + NW * i) * 1024);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 16 / NW; ++i) {
       const int w = wave + NW * i;
@@ -329,9 +359,15 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       __builtin_amdgcn_global_load_lds(src, (lds_vp)(base + w * 1024), 16, 0, 0);
     }
   };
-  auto issueV = [&](int j) {  // 16 wave loads of 8 V^T rows x 128 B, 2 per wave
+  auto issueV = [&](int j) {  // 16 wave loads (one slot of 4 rows, or 8 V^T rows x 128 B), 16 / NW per wave
     const int k0 = j * BN;
     char* base = vring + (j & 1) * VST;
+    if constexpr (VR) {
+      const int n = bytes(j);
+#pragma unroll
+      for (int i = 0; i < 16 / NW; ++i) buffer_to_lds(Vb + k0 * kl.s, n, vvo[i], base + (wave + NW * i) * kSlot);
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 16 / NW; ++i) {
       const int w = wave + NW * i;
@@ -353,7 +389,13 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   for (int ks = 0; ks < 4; ++ks) koff[ks] = krow0 * 256 + (((4 * ks + G) ^ r16) << 4);
   int voff[2];
 #pragma unroll
-  for (int kc = 0; kc < 2; ++kc) voff[kc] = r16 * 128 + (((4 * kc + G) ^ vswz3(r16)) << 4);
+  for (int kc = 0; kc < 2; ++kc)  // VR: keys kbase + r16 / 4 (+ 8), dims 4 (r16 % 4) .. + 3
+    voff[kc] = VR ? (4 * (G & 1) + (r16 >> 2)) * kSlot + (G >> 1) * 256 + 8 * (r16 & 3) + kc * 512
+                  : r16 * 128 + (((4 * kc + G) ^ vswz3(r16)) << 4);
+  auto vfrag = [&](const char* vb, int kc, int dt) {
+    if constexpr (VR) return lds_frag_tr(vb + voff[kc] + dt * 32, 8 * kSlot);
+    else return *reinterpret_cast<const i32x4*>(vb + voff[kc] + dt * 16 * 128);
+  };
   constexpr int ktoff[4] = {0, 8 * 256, 32 * 256, 40 * 256};
 
   f32x4 S[4][2];
@@ -390,7 +432,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
-        const i32x4 a = *reinterpret_cast<const i32x4*>(vb + voff[kc] + dt * 16 * 128);
+        const i32x4 a = vfrag(vb, kc, dt);
 #pragma unroll
         for (int u = 0; u < 2; ++u) oacc[dt][u] = mma16<T>(as_frag(a), as_frag(P[u][kc]), oacc[dt][u]);
       }
@@ -482,7 +524,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int dd = 0; dd < 2; ++dd)
 #pragma unroll
           for (int kc = 0; kc < 2; ++kc)
-            F[2 * dd + kc] = *reinterpret_cast<const i32x4*>(vb + voff[kc] + (2 * st + dd) * 16 * 128);
+            F[2 * dd + kc] = vfrag(vb, kc, 2 * st + dd);
       } else {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) F[kt] = *reinterpret_cast<const i32x4*>(kb + koff[st - 4] + ktoff[kt]);
@@ -582,7 +624,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
       u16* orow = O + b * ql.b + h * ql.h + (int64_t)qi * ql.s;
 #pragma unroll
       for (int dt = 0; dt < 8; ++dt) {
-        typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
         i32x2 w;
         w[0] = (int)pack2<T>(oacc[dt][u][0] * inv, oacc[dt][u][1] * inv);
         w[1] = (int)pack2<T>(oacc[dt][u][2] * inv, oacc[dt][u][3] * inv);
@@ -594,15 +635,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 }
 
 // ============================================================================ backward, D = 128 (MFMA 16x16x32)
-// 8 bytes from LDS with the gfx950 transpose read: within each 16-lane group, lane j receives
-// element j % 4 of the 8-byte pieces addressed by lanes j / 4 + 4 k, k = 0..3.  Two such reads, by
-// lanes addressing rows k0 + i / 4 (+ 4) at columns m0 + 4 (i % 4), return the MFMA fragment
+// Two LDS transpose reads, by lanes addressing rows k0 + i / 4 (+ 4) at columns m0 + 4 (i % 4), return the MFMA fragment
 // A[m0 + j][k0 .. k0 + 7] of a row-major [k][m] tile: the transposed operand without a copy.
-typedef short v4s_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
-Q3_DEV i32x2 ldtr(const char* p) {
-  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s_t*)p));
-}
+Q3_DEV i32x2 ldtr(const char* p) { return lds_read_tr((lds_v4s)p); }
 // 16-byte chunk swizzle of the 256-byte query rows of the dK/dV tiles: a bijection onto 0..15 of
 // the 16 rows a row-read pass touches ({0-3, 8-11, 16-19, 24-27}, +4), and distinct 32-byte bank
 // groups for the 8 rows of each half-wave pass of a transpose read.
@@ -795,15 +830,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // through a 2-stage direct-to-LDS ring.  Per block: S^T = K Q^T, dP^T = V dO^T (Q, dO fragments in
 // registers), P^T = exp2(S^T s - lse), dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T; the K/V row
 // mapping of the forward makes dS^T the B operand of the K^T product as it comes out.
+// The K tile is laid out in the slots of the forward's V tile (chunks of the odd 16-key rows swapped in pairs), which
+// serve the row reads of S = K Q^T and the transpose reads of dQ^T += K^T dS^T alike: no K^T copy, a third less LDS
+// traffic (backward, B4 S2048 566 -> 546 us, B3 S1000 fp16 148 -> 136, B2 S512 74 -> 67, S8192 within 0.6 %).  delta = rowsum(O dO) is formed here from the dO fragments in registers and written for the dK/dV kernel
+// (O null: read from Delta instead).
 template <typename T, int GH>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_bwd_dq_v3(
     const u16* __restrict__ Q, Lay ql, const u16* __restrict__ K, const u16* __restrict__ V, Lay kl,
-    const u16* __restrict__ Kt, const u16* __restrict__ dO, const float* __restrict__ LSE,
-    const float* __restrict__ Delta, u16* __restrict__ dQ, int Hq, int Hkv, int Lq, int Lk, int ldkt, float scale,
-    float scale2) {
+    const u16* __restrict__ O, const u16* __restrict__ dO, const float* __restrict__ LSE, float* Delta,
+    u16* __restrict__ dQ, int Hq, int Hkv, int Lq, int Lk, float scale, float scale2) {
   constexpr int D = 128, BN = 64, NW = 8, QT = 32 * (NW / GH);
-  constexpr int KST = BN * D * 2;  // one 64 x 128 tile
-  constexpr int STAGE = 3 * KST;   // K, V, K^T
+  constexpr int STAGE = kRowTile + BN * D * 2;  // K, V
   __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
 
   const int nqt = (Lq + QT - 1) / QT;
@@ -816,7 +853,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int q0 = qt * QT + (wave / GH) * 32;
   const u16* Kb = K + b * kl.b + hk * kl.h;
   const u16* Vb = V + b * kl.b + hk * kl.h;
-  const u16* Ktb = Kt + (int64_t)(b * Hkv + hk) * D * ldkt;
 
   bf16x8_t qf[2][4], df[2][4];
   float lse2[2], dlt[2];
@@ -830,7 +866,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       df[u][ks] = as_frag(ld16(dO + row + 32 * ks + 8 * G));
     }
     lse2[u] = LSE[(int64_t)bh * Lq + qi] * kLog2e;
-    dlt[u] = Delta[(int64_t)bh * Lq + qi];
+    if (O) {
+      float sum = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const Vec<T> o = load_vec<T>(O + row + 32 * ks + 8 * G), g = unpack_vec<T>(__builtin_bit_cast(i32x4, df[u][ks]));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum += o.v[e] * g.v[e];
+      }
+      sum += __shfl_xor(sum, 16, 64);
+      sum += __shfl_xor(sum, 32, 64);
+      dlt[u] = sum;
+      if (G == 0 && q0 + 16 * u + r16 < Lq) Delta[(int64_t)bh * Lq + qi] = sum;
+    } else {
+      dlt[u] = Delta[(int64_t)bh * Lq + qi];
+    }
   }
 
   const int nb = (min(Lk, min(qt * QT + QT - 1, Lq - 1) + off + 1) + BN - 1) / BN;
@@ -838,33 +888,32 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int nfull = min(nbw, max(0, (q0 + off + 1) / BN));  // blocks fully visible to the wave
   const int qpos[2] = {q0 + r16 + off, q0 + 16 + r16 + off};
 
-  auto issue = [&](int j) {  // K, V: 16 wave loads each (4 rows x 256 B); K^T: 16 (8 rows x 128 B)
+  auto issue = [&](int j) {  // K, V: 16 wave loads each (4 rows x 256 B)
     const int k0 = j * BN;
     char* base = lds + (j & 1) * STAGE;
 #pragma unroll
     for (int i = 0; i < 16 / NW; ++i) {
       const int w = wave + NW * i;
-      const int r = w * 4 + (lane >> 4);
+      const int sub = lane >> 4;
+      __builtin_amdgcn_global_load_lds(Kb + (int64_t)min(k0 + w + 16 * sub, Lk - 1) * kl.s + ((lane & 15) ^ (sub & 1)) * 8,
+                                       (lds_vp)(base + w * kSlot), 16, 0, 0);
+      const int r = w * 4 + sub;
       const int c = (lane & 15) ^ kswz3(r);
-      const int64_t src = (int64_t)min(k0 + r, Lk - 1) * kl.s + c * 8;
-      __builtin_amdgcn_global_load_lds(Kb + src, (lds_vp)(base + w * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(Vb + src, (lds_vp)(base + KST + w * 1024), 16, 0, 0);
-      const int rt = w * 8 + (lane >> 3);
-      const int ct = (lane & 7) ^ vswz3(rt);
-      __builtin_amdgcn_global_load_lds(Ktb + (int64_t)rt * ldkt + min(k0 + ct * 8, ldkt - 8),
-                                       (lds_vp)(base + 2 * KST + w * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(Vb + (int64_t)min(k0 + r, Lk - 1) * kl.s + c * 8,
+                                       (lds_vp)(base + kRowTile + w * 1024), 16, 0, 0);
     }
   };
 
   const int krow0 = 4 * ((r16 >> 2) & 1) + 16 * (r16 >> 3) + (r16 & 3);
   const int kbase = 4 * (G & 1) + 16 * (G >> 1);
-  int koff[4];
+  int koff[4], vrow[4];
 #pragma unroll
-  for (int ks = 0; ks < 4; ++ks) koff[ks] = krow0 * 256 + (((4 * ks + G) ^ r16) << 4);
-  int toff[2];
-#pragma unroll
-  for (int kc = 0; kc < 2; ++kc) toff[kc] = r16 * 128 + (((4 * kc + G) ^ vswz3(r16)) << 4);
-  constexpr int ktoff[4] = {0, 8 * 256, 32 * 256, 40 * 256};
+  for (int ks = 0; ks < 4; ++ks) {
+    koff[ks] = (r16 & 7) * kSlot + (r16 >> 3) * 256 + (((4 * ks + G) ^ (r16 >> 3)) << 4);
+    vrow[ks] = kRowTile + krow0 * 256 + (((4 * ks + G) ^ r16) << 4);
+  }
+  const int toff = (4 * (G & 1) + (r16 >> 2)) * kSlot + (G >> 1) * 256 + ((((r16 >> 1) & 1) ^ (G >> 1)) << 4) + 8 * (r16 & 1);
+  constexpr int ktoff[4] = {0, 8 * kSlot, 512, 8 * kSlot + 512}, vtoff[4] = {0, 8 * 256, 32 * 256, 40 * 256};
 
   f32x4 dq[8][2];
 #pragma unroll
@@ -881,15 +930,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (j + 1 < nb) issue(j + 1);
     if (j >= nbw) continue;
     const char* kb = lds + (j & 1) * STAGE;
-    const char* vb = kb + KST;
-    const char* tb = kb + 2 * KST;
     f32x4 S[4][2], DP[4][2];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks)
 #pragma unroll
       for (int kt = 0; kt < 4; ++kt) {
         const i32x4 a = *reinterpret_cast<const i32x4*>(kb + koff[ks] + ktoff[kt]);
-        const i32x4 av = *reinterpret_cast<const i32x4*>(vb + koff[ks] + ktoff[kt]);
+        const i32x4 av = *reinterpret_cast<const i32x4*>(kb + vrow[ks] + vtoff[kt]);
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           S[kt][u] = mma16<T>(as_frag(a), qf[u][ks], ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : S[kt][u]);
@@ -923,7 +970,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     for (int dt = 0; dt < 8; ++dt)
 #pragma unroll
       for (int kc = 0; kc < 2; ++kc) {
-        const i32x4 a = *reinterpret_cast<const i32x4*>(tb + toff[kc] + dt * 16 * 128);
+        const i32x4 a = lds_frag_tr(kb + toff + kc * 512 + dt * 32, 8 * kSlot);
 #pragma unroll
         for (int u = 0; u < 2; ++u) dq[dt][u] = mma16<T>(as_frag(a), as_frag(DS[u][kc]), dq[dt][u]);
       }
@@ -1123,7 +1170,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int vg = 0; vg < 4; ++vg) {
         const int d = dt * 32 + 8 * vg + 4 * g;
-        typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
         i32x2 w;
         w[0] = (int)pack2<T>(dq[dt][4 * vg] * scale, dq[dt][4 * vg + 1] * scale);
         w[1] = (int)pack2<T>(dq[dt][4 * vg + 2] * scale, dq[dt][4 * vg + 3] * scale);
@@ -1361,7 +1407,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(OCC, O
 #pragma unroll
       for (int vg = 0; vg < 4; ++vg) {
         const int d = dt * 32 + 8 * vg + 4 * g;
-        typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
         i32x2 wk, wv;
         wk[0] = (int)pack2<T>(dk[dt][4 * vg] * scale, dk[dt][4 * vg + 1] * scale);
         wk[1] = (int)pack2<T>(dk[dt][4 * vg + 2] * scale, dk[dt][4 * vg + 3] * scale);
@@ -1579,13 +1624,18 @@ __global__ __launch_bounds__(kThreads) void seq_major_vec_kernel(const u16* __re
 // ============================================================================ host dispatch
 bool dtype_ok(int dt) { return dt == Q3_F32 || dt == Q3_F16 || dt == Q3_BF16; }
 
+// v: V's rows (ldvt 0) or the sequence-major copy.
 template <typename T, int GH, int NW>
-int fwd_v3_launch(const void* q, Lay ql, const void* k, Lay kl, const void* vt, void* o, float* lse, int B, int Hq,
+int fwd_v3_launch(const void* q, Lay ql, const void* k, Lay kl, const void* v, void* o, float* lse, int B, int Hq,
                   int Hkv, int Lq, int Lk, int ldvt, float scale, hipStream_t s) {
   constexpr int QT = 32 * (NW / GH);
   dim3 grid((unsigned)(B * Hq / GH), (unsigned)((Lq + QT - 1) / QT));
-  attn_fwd_v3<T, GH, NW><<<grid, NW * 64, 0, s>>>((const u16*)q, ql, (const u16*)k, kl, (const u16*)vt, (u16*)o,
-                                                  lse, Hq, Hkv, Lq, Lk, ldvt, scale * kLog2e);
+  if (ldvt == 0)
+    attn_fwd_v3<T, GH, NW, true><<<grid, NW * 64, 0, s>>>((const u16*)q, ql, (const u16*)k, kl, (const u16*)v, (u16*)o,
+                                                          lse, Hq, Hkv, Lq, Lk, 0, scale * kLog2e);
+  else
+    attn_fwd_v3<T, GH, NW, false><<<grid, NW * 64, 0, s>>>((const u16*)q, ql, (const u16*)k, kl, (const u16*)v, (u16*)o,
+                                                           lse, Hq, Hkv, Lq, Lk, ldvt, scale * kLog2e);
   return (int)hipGetLastError();
 }
 
@@ -1630,29 +1680,29 @@ int q3i_attn_bwd_dkdv_v4(int dtype, const void* q, int64_t qsb, int64_t qsh, int
 namespace {
 
 template <typename T, int GH>
-int bwd_dq_v3(const void* q, Lay ql, const void* k, const void* v, Lay kl, const void* kt, const void* dout,
-              const float* lse, const float* delta, void* dq, int B, int Hq, int Hkv, int Lq, int Lk, int ldkt,
-              float scale, hipStream_t s) {
+int bwd_dq_v3(const void* q, Lay ql, const void* k, const void* v, Lay kl, const void* o, const void* dout,
+              const float* lse, float* delta, void* dq, int B, int Hq, int Hkv, int Lq, int Lk, float scale,
+              hipStream_t s) {
   constexpr int QT = 32 * (8 / GH);
   dim3 g((unsigned)(B * Hq / GH), (unsigned)((Lq + QT - 1) / QT));
-  attn_bwd_dq_v3<T, GH><<<g, 512, 0, s>>>((const u16*)q, ql, (const u16*)k, (const u16*)v, kl, (const u16*)kt,
-                                          (const u16*)dout, lse, delta, (u16*)dq, Hq, Hkv, Lq, Lk, ldkt, scale,
+  attn_bwd_dq_v3<T, GH><<<g, 512, 0, s>>>((const u16*)q, ql, (const u16*)k, (const u16*)v, kl, (const u16*)o,
+                                          (const u16*)dout, lse, delta, (u16*)dq, Hq, Hkv, Lq, Lk, scale,
                                           scale * kLog2e);
   return (int)hipGetLastError();
 }
 
 template <typename T, int D>
-int bwd_mfma(const void* q, Lay ql, const void* k, const void* v, Lay kl, const void* qt, const void* kt,
-             const void* dout, const void* dot, const float* lse, const float* delta, void* dq, void* dk, void* dv,
-             int B, int Hq, int Hkv, int Lq, int Lk, int ldqt, int ldkt, float scale, hipStream_t s) {
+int bwd_mfma(const void* q, Lay ql, const void* k, const void* v, Lay kl, const void* o, const void* qt,
+             const void* kt, const void* dout, const void* dot, const float* lse, float* delta, void* dq, void* dk,
+             void* dv, int B, int Hq, int Hkv, int Lq, int Lk, int ldqt, int ldkt, float scale, hipStream_t s) {
   if constexpr (D == 128) {
-    // dQ on 8-wave GQA workgroups (K^T copy), dK/dV with transpose reads (qt, dot unused)
+    // dQ on 8-wave GQA workgroups, then dK/dV, both with transpose reads (the copies are unused); o set: dQ
+    // forms delta
     const int grp = Hq / Hkv;
     int rc;
-    if (grp % 4 == 0) rc = bwd_dq_v3<T, 4>(q, ql, k, v, kl, kt, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, ldkt, scale, s);
-    else if (grp % 2 == 0)
-      rc = bwd_dq_v3<T, 2>(q, ql, k, v, kl, kt, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, ldkt, scale, s);
-    else rc = bwd_dq_v3<T, 1>(q, ql, k, v, kl, kt, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, ldkt, scale, s);
+    if (grp % 4 == 0) rc = bwd_dq_v3<T, 4>(q, ql, k, v, kl, o, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, scale, s);
+    else if (grp % 2 == 0) rc = bwd_dq_v3<T, 2>(q, ql, k, v, kl, o, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, scale, s);
+    else rc = bwd_dq_v3<T, 1>(q, ql, k, v, kl, o, dout, lse, delta, dq, B, Hq, Hkv, Lq, Lk, scale, s);
     if (rc) return rc;
     // one query head per wave, 48-key wave tiles (attention_bwd.hip): its buffer descriptors hold 32-bit tile offsets
     // and count a head's rows in 32-bit units of 16 bytes; wider operands take the kernel below, as other groups do
@@ -1767,8 +1817,12 @@ int q3_attention_fwd(int dtype, const void* q, int64_t qsb, int64_t qsh, int64_t
   const Lay ql{qsb, qsh, qss}, kl{ksb, ksh, kss};
   const int b = (int)B, hq = (int)Hq, hkv = (int)Hkv, lq = (int)Lq, lk = (int)Lk;
   if (q3_attention_mfma_supported(dtype, D)) {
-    Q3_REQUIRE(vt && ldvt >= Lk && ldvt % 16 == 0 && lay_ok(q, ql) && lay_ok(k, kl) && lay_ok(o, ql) && al16(vt));
-    const int ld = (int)ldvt;
+    // D = 128 reads V's rows where they are 16-byte aligned and within the descriptors' 32-bit offsets; otherwise the sequence-major copy is needed
+    const bool rows = D == 128 && v && lay_ok(v, kl) && kl.s < (1 << 24);
+    Q3_REQUIRE(lay_ok(q, ql) && lay_ok(k, kl) && lay_ok(o, ql));
+    Q3_REQUIRE(rows || (vt && ldvt >= Lk && ldvt % 16 == 0 && al16(vt)));
+    const int ld = rows ? 0 : (int)ldvt;
+    if (rows) vt = v;
     if (dtype == Q3_BF16) return Q3_ATTN_D(BF16, fwd_mfma, q, ql, k, kl, vt, o, lse, b, hq, hkv, lq, lk, ld, scale, stream);
     return Q3_ATTN_D(F16, fwd_mfma, q, ql, k, kl, vt, o, lse, b, hq, hkv, lq, lk, ld, scale, stream);
   }
@@ -1787,22 +1841,28 @@ int q3_attention_bwd(int dtype, const void* q, int64_t qsb, int64_t qsh, int64_t
              shapes_ok(B, Hq, Hkv, Lq, Lk, D));
   const Lay ql{qsb, qsh, qss}, kl{ksb, ksh, kss};
   const int b = (int)B, hq = (int)Hq, hkv = (int)Hkv, lq = (int)Lq, lk = (int)Lk, d = (int)D;
-  int rc;
-  if (dtype == Q3_BF16) rc = delta_t<BF16>(o, dout, ql, delta, B * Hq * Lq, hq, lq, d, stream);
-  else if (dtype == Q3_F16) rc = delta_t<F16>(o, dout, ql, delta, B * Hq * Lq, hq, lq, d, stream);
-  else rc = delta_t<F32>(o, dout, ql, delta, B * Hq * Lq, hq, lq, d, stream);
-  if (rc) return rc;
+  // D = 128 on the matrix cores: the dQ kernel forms delta itself (16-byte aligned O rows)
+  const bool own_delta = D == 128 && q3_attention_mfma_supported(dtype, D) && lay_ok(o, ql);
+  if (!own_delta) {
+    int rc;
+    if (dtype == Q3_BF16) rc = delta_t<BF16>(o, dout, ql, delta, B * Hq * Lq, hq, lq, d, stream);
+    else if (dtype == Q3_F16) rc = delta_t<F16>(o, dout, ql, delta, B * Hq * Lq, hq, lq, d, stream);
+    else rc = delta_t<F32>(o, dout, ql, delta, B * Hq * Lq, hq, lq, d, stream);
+    if (rc) return rc;
+  }
   if (q3_attention_mfma_supported(dtype, D)) {
-    // D = 128 reads Q and dO transposed straight from LDS: qt / dot are not needed (may be null)
-    const bool need_qt = D != 128;
-    Q3_REQUIRE(kt && ldkt >= Lk && ldkt % 16 == 0 && lay_ok(q, ql) && lay_ok(dout, ql) && lay_ok(dq, ql) &&
-               lay_ok(k, kl) && lay_ok(v, kl) && lay_ok(dk, kl) && lay_ok(dv, kl) && al16(kt));
-    Q3_REQUIRE(!need_qt || (qt && dot && ldqt >= Lq && ldqt % 16 == 0 && al16(qt) && al16(dot)));
+    // D = 128 reads K, Q and dO transposed straight from LDS: kt / qt / dot are not needed (may be null)
+    const bool copies = D != 128;
+    Q3_REQUIRE(lay_ok(q, ql) && lay_ok(dout, ql) && lay_ok(dq, ql) && lay_ok(k, kl) && lay_ok(v, kl) &&
+               lay_ok(dk, kl) && lay_ok(dv, kl));
+    Q3_REQUIRE(!copies || (kt && qt && dot && ldkt >= Lk && ldkt % 16 == 0 && al16(kt) && ldqt >= Lq &&
+                           ldqt % 16 == 0 && al16(qt) && al16(dot)));
     const int lq8 = (int)ldqt, lk8 = (int)ldkt;
+    const void* od = own_delta ? o : nullptr;
     if (dtype == Q3_BF16)
-      return Q3_ATTN_D(BF16, bwd_mfma, q, ql, k, v, kl, qt, kt, dout, dot, lse, delta, dq, dk, dv, b, hq, hkv, lq, lk,
+      return Q3_ATTN_D(BF16, bwd_mfma, q, ql, k, v, kl, od, qt, kt, dout, dot, lse, delta, dq, dk, dv, b, hq, hkv, lq, lk,
                        lq8, lk8, scale, stream);
-    return Q3_ATTN_D(F16, bwd_mfma, q, ql, k, v, kl, qt, kt, dout, dot, lse, delta, dq, dk, dv, b, hq, hkv, lq, lk,
+    return Q3_ATTN_D(F16, bwd_mfma, q, ql, k, v, kl, od, qt, kt, dout, dot, lse, delta, dq, dk, dv, b, hq, hkv, lq, lk,
                      lq8, lk8, scale, stream);
   }
   if (dtype == Q3_BF16)

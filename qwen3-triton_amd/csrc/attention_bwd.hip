@@ -19,8 +19,6 @@
 
 namespace {
 
-typedef short v4s_t __attribute__((ext_vector_type(4)));
-typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
 typedef __attribute__((address_space(3))) void* lds_vp;
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -33,14 +31,7 @@ static_assert(4 * kRed <= 4 * kWaveLds, "the fold reuses the rings");
 
 Q3_DEV i32x4 ld16(const u16* p) { return *reinterpret_cast<const i32x4*>(p); }
 Q3_DEV bf16x8_t as_frag(i32x4 v) { return __builtin_bit_cast(bf16x8_t, v); }
-// 8 bytes by the gfx950 transpose read: within each 16-lane group, lane j receives element j % 4 of
-// the 8-byte pieces addressed by lanes j / 4 + 4 k, k = 0..3.  Read through a __restrict parameter: without alias
-// information the compiler waits for every direct-to-LDS load in flight before such a read.
-typedef __attribute__((address_space(3))) v4s_t* lds_v4s;
-Q3_DEV i32x2 ldtr_at(lds_v4s __restrict p) {
-  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p));
-}
-Q3_DEV i32x2 ldtr(const char* p) { return ldtr_at((lds_v4s)p); }
+Q3_DEV i32x2 ldtr(const char* p) { return lds_read_tr((lds_v4s)p); }
 // 16-byte chunk swizzle of the 256-byte query rows: conflict-free row reads (16 rows of one chunk
 // column) and distinct 32-byte bank groups for the 8 rows of each half-wave transpose read.
 Q3_DEV int qswz(int r) { return 2 * ((r & 3) | (((r >> 3) & 1) << 2)) + ((r >> 4) & 1); }

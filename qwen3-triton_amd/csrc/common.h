@@ -114,6 +114,25 @@ template <> Q3_DEV f32x4 mfma_16x16x32<F16>(bf16x8_t a, bf16x8_t b, f32x4 c) {
                                                  0, 0, 0);
 }
 
+// ------------------------------------------------------------------ LDS transpose read
+// 8 bytes by the gfx950 transpose read: within each 16-lane group, lane j receives element j % 4 of the
+// 8-byte pieces addressed by lanes j / 4 + 4 k, k = 0..3.
+// The read goes through a __restrict parameter: that gives the instruction alias information, without which
+// the compiler assumes it may read the target of any direct-to-LDS load in flight and waits for all of them
+// (s_waitcnt vmcnt(0)) first, emptying the ring.  Ordering against the ring is each kernel's own wait, as for
+// its ordinary LDS reads.
+typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
+typedef short v4s_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) v4s_t* lds_v4s;
+Q3_DEV i32x2 lds_read_tr(lds_v4s __restrict p) {
+  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p));
+}
+// Two such reads, `step` bytes apart: one 16-byte MFMA fragment.
+Q3_DEV i32x4 lds_frag_tr(const char* p, int step) {
+  const i32x2 lo = lds_read_tr((lds_v4s)p), hi = lds_read_tr((lds_v4s)(p + step));
+  return i32x4{lo[0], lo[1], hi[0], hi[1]};
+}
+
 // ------------------------------------------------------------------ wave64 reductions
 // Butterfly over aligned groups of WIDTH lanes (WIDTH a power of two <= 64); every lane in
 // the group ends with the full result.  Offsets 1/2 use DPP quad permutes, 4/8 DPP row

@@ -21,20 +21,6 @@
 
 namespace q3gemm {
 
-typedef __attribute__((__vector_size__(2 * sizeof(int)))) int i32x2;
-typedef short v4s __attribute__((ext_vector_type(4)));
-
-// 8 bytes by the gfx950 transpose read: within each 16-lane group, lane j receives element j % 4 of the
-// 8-byte pieces addressed by lanes j / 4 + 4 k, k = 0..3.
-// The read goes through a __restrict parameter: that gives the instruction alias information, without which
-// the compiler assumes it may read the target of any direct-to-LDS load in flight and waits for all of them
-// (s_waitcnt vmcnt(0)) first, emptying the ring.  Ordering against the ring is ring_sync's, as for ordinary
-// LDS reads.
-typedef __attribute__((address_space(3))) v4s* lds_v4s;
-Q3_DEV i32x2 lds_read_tr(lds_v4s __restrict p) {
-  return __builtin_bit_cast(i32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(p));
-}
-
 // Workgroup barrier for a direct-to-LDS ring: this wave's loads older than its newest N have landed in
 // LDS and its own LDS reads are done (vmcnt(N) lgkmcnt(0)), then s_barrier.  __syncthreads() would drain
 // every prefetched stage of the ring at each k-tile.
@@ -270,10 +256,7 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
     fb[ks] = ABYTES + frag_base(BT, BN, wn * TNW, ks) + (BT ? ks * 512 : 0);
   }
   bf16x8_t af[2][FM], bfr[2][FN];
-  auto tread = [&](const char* p) {
-    const i32x2 lo = lds_read_tr((lds_v4s)p), hi = lds_read_tr((lds_v4s)(p + kSlot4));
-    return __builtin_bit_cast(bf16x8_t, i32x4{lo[0], lo[1], hi[0], hi[1]});
-  };
+  auto tread = [&](const char* p) { return __builtin_bit_cast(bf16x8_t, lds_frag_tr(p, kSlot4)); };
   auto load = [&](int stage, int buf, int ks) {
     const char* sb = lds + stage * STAGE;
 #pragma unroll

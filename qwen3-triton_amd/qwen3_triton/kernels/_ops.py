@@ -272,8 +272,9 @@ def attention_fwd(q, k, v, scale):
         o = torch.empty_strided(q.shape, q.stride(), device=q.device, dtype=q.dtype)
     lse = torch.empty((b, hq, lq), device=q.device, dtype=torch.float32)
     vt, ldvt = None, 0
-    if attention_mfma(q.dtype, d):
-        vt = seq_major(v)
+    if attention_mfma(q.dtype, d) and not (d == 128 and v.data_ptr() % 16 == 0 and
+                                           all(st % 8 == 0 for st in v.stride()[:3]) and v.stride(2) < 1 << 24):
+        vt = seq_major(v)   # head_dim 128 reads aligned rows of V as they lie (32-bit tile offsets)
         ldvt = vt.shape[-1]
     H.call("q3_attention_fwd", H.code(q.dtype), q.data_ptr(), *_bhsd_strides(q), k.data_ptr(), v.data_ptr(),
            *_bhsd_strides(k), 0 if vt is None else vt.data_ptr(), ldvt, o.data_ptr(), lse.data_ptr(), b, hq, hkv,
@@ -301,12 +302,9 @@ def attention_bwd(q, k, v, o, lse, do, scale):
     delta = torch.empty((b, hq, lq), device=q.device, dtype=torch.float32)
     qt = kt = dot = None
     ldq = ldk = 0
-    if attention_mfma(q.dtype, d):
-        kt = seq_major(k)
-        ldk = kt.shape[-1]
-        if d != 128:  # head_dim 128 reads Q and dO transposed in LDS
-            qt, dot = seq_major(q), seq_major(do)
-            ldq = qt.shape[-1]
+    if d != 128 and attention_mfma(q.dtype, d):  # head_dim 128 reads K, Q and dO transposed in LDS
+        kt, qt, dot = seq_major(k), seq_major(q), seq_major(do)
+        ldk, ldq = kt.shape[-1], qt.shape[-1]
     p = (lambda t: 0 if t is None else t.data_ptr())
     H.call("q3_attention_bwd", H.code(q.dtype), q.data_ptr(), *_bhsd_strides(q), k.data_ptr(), v.data_ptr(),
            *_bhsd_strides(k), o.data_ptr(), do.data_ptr(), lse.data_ptr(), p(qt), ldq, p(kt), ldk, p(dot),

@@ -199,3 +199,27 @@ def test_attention_wide_position_stride():
     for a, x, n in zip(grads, e, "qkv"):
         assert cosine(a, x) >= 0.999, f"d{n} cosine"
         assert max_rel(a, x) <= GRAD_TOL[torch.bfloat16], f"d{n} max-rel {max_rel(a, x)}"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("hq,hk,lq,lk", [(4, 4, 1, 1), (4, 2, 7, 63), (8, 2, 65, 65), (16, 4, 33, 129), (4, 1, 128, 256)])
+def test_attention_value_rows_and_copies_agree(hq, hk, lq, lk, dtype):
+    """head_dim 128: V read as its rows lie and through the sequence-major copy (V off 16-byte alignment by one
+    element) multiply the same values in the same order: equal bits, in both memory orders, the rows around the
+    operands holding NaN."""
+    print(f"attention value routes {hq} {hk} {lq} {lk} {dtype}", flush=True)
+    q, k, v, _ = make(2, hq, hk, lq, lk, 128, dtype, seed=lq + lk)
+    for order in ((0, 1, 2), (0, 2, 1)):            # [B,H,L,D] and [B,L,H,D] memory
+        def lay(t, off):
+            dims = [t.shape[i] for i in order]
+            flat = torch.full((t.numel() + 256 + off,), float("nan"), dtype=dtype, device="cuda")
+            x = flat[128 + off:128 + off + t.numel()].view(*dims, 128).permute(*order, 3)
+            x.copy_(t)
+            return x
+        qd, kd = lay(q, 0), lay(k, 0)
+        rows, copied = lay(v, 0), lay(v, 1)
+        assert rows.data_ptr() % 16 == 0 and copied.data_ptr() % 16 != 0
+        o, lse = _ops.attention_fwd(qd, kd, rows, 128 ** -0.5)
+        oc, lsec = _ops.attention_fwd(qd, kd, copied, 128 ** -0.5)
+        assert bool(torch.isfinite(o).all())
+        assert torch.equal(o, oc) and torch.equal(lse, lsec)
