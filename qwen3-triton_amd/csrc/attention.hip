@@ -834,7 +834,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
 // serve the row reads of S = K Q^T and the transpose reads of dQ^T += K^T dS^T alike: no K^T copy, a third less LDS
 // traffic (backward, B4 S2048 566 -> 546 us, B3 S1000 fp16 148 -> 136, B2 S512 74 -> 67, S8192 within 0.6 %).  delta = rowsum(O dO) is formed here from the dO fragments in registers and written for the dK/dV kernel
 // (O null: read from Delta instead).
-template <typename T, int GH>
+template <typename T, int GH, bool DESC>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_bwd_dq_v3(
     const u16* __restrict__ Q, Lay ql, const u16* __restrict__ K, const u16* __restrict__ V, Lay kl,
     const u16* __restrict__ O, const u16* __restrict__ dO, const float* __restrict__ LSE, float* Delta,
@@ -888,12 +888,26 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int nfull = min(nbw, max(0, (q0 + off + 1) / BN));  // blocks fully visible to the wave
   const int qpos[2] = {q0 + r16 + off, q0 + 16 + r16 + off};
 
+  // Descriptors as in the forward (DESC: 32-bit tile offsets reach kl); otherwise an address per load, which took the
+  // backward at B1 S8192 1902 us against 1864, B4 S2048 545 against 541, B2 S512 67.5 against 66.5.
+  uint32_t kvo[16 / NW], vvo[16 / NW];
+#pragma unroll
+  for (int i = 0; i < 16 / NW; ++i) {
+    const int w = wave + NW * i, sub = lane >> 4, r = 4 * w + sub;
+    kvo[i] = (uint32_t)(((w + 16 * sub) * (int)kl.s + ((lane & 15) ^ (sub & 1)) * 8) * 2);
+    vvo[i] = (uint32_t)((r * (int)kl.s + ((lane & 15) ^ kswz3(r)) * 8) * 2);
+  }
   auto issue = [&](int j) {  // K, V: 16 wave loads each (4 rows x 256 B)
-    const int k0 = j * BN;
+    const int k0 = j * BN, n = (min(Lk - k0, BN) - 1) * ((int)kl.s * 2) + 2 * D;
     char* base = lds + (j & 1) * STAGE;
 #pragma unroll
     for (int i = 0; i < 16 / NW; ++i) {
       const int w = wave + NW * i;
+      if constexpr (DESC) {
+        buffer_to_lds(Kb + k0 * kl.s, n, kvo[i], base + w * kSlot);
+        buffer_to_lds(Vb + k0 * kl.s, n, vvo[i], base + kRowTile + w * 1024);
+        continue;
+      }
       const int sub = lane >> 4;
       __builtin_amdgcn_global_load_lds(Kb + (int64_t)min(k0 + w + 16 * sub, Lk - 1) * kl.s + ((lane & 15) ^ (sub & 1)) * 8,
                                        (lds_vp)(base + w * kSlot), 16, 0, 0);
@@ -1685,7 +1699,12 @@ int bwd_dq_v3(const void* q, Lay ql, const void* k, const void* v, Lay kl, const
               hipStream_t s) {
   constexpr int QT = 32 * (8 / GH);
   dim3 g((unsigned)(B * Hq / GH), (unsigned)((Lq + QT - 1) / QT));
-  attn_bwd_dq_v3<T, GH><<<g, 512, 0, s>>>((const u16*)q, ql, (const u16*)k, (const u16*)v, kl, (const u16*)o,
+  if (kl.s < (1 << 24))  // as for the forward's V rows
+    attn_bwd_dq_v3<T, GH, true><<<g, 512, 0, s>>>((const u16*)q, ql, (const u16*)k, (const u16*)v, kl, (const u16*)o,
+                                          (const u16*)dout, lse, delta, (u16*)dq, Hq, Hkv, Lq, Lk, scale,
+                                          scale * kLog2e);
+  else
+    attn_bwd_dq_v3<T, GH, false><<<g, 512, 0, s>>>((const u16*)q, ql, (const u16*)k, (const u16*)v, kl, (const u16*)o,
                                           (const u16*)dout, lse, delta, (u16*)dq, Hq, Hkv, Lq, Lk, scale,
                                           scale * kLog2e);
   return (int)hipGetLastError();
