@@ -290,6 +290,9 @@ typedef struct q3_gemm_desc {
   float eps;
 } q3_gemm_desc;
 size_t q3_gemm_workspace_bytes(const q3_gemm_desc* desc);
+/* The launches that q3_gemm makes for desc (host only, nothing runs): their number (1 or 2; 0: refused), and per
+ * launch {first row, rows, tile rows, tile columns, k splits} in out[0..4] and out[5..9]. */
+int q3_gemm_plan(const q3_gemm_desc* desc, int64_t* out);
 int q3_gemm(const q3_gemm_desc* desc, void* workspace, size_t workspace_bytes, hipStream_t stream);
 /* Same product for arbitrary element strides: A(m,k) = A[m*sam + k*sak], B(k,n) = B[k*sbk + n*sbn];
  * any dtype (fp32 included).  SIMT path for shapes the matrix-core kernel does not take.

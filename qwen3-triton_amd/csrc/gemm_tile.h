@@ -56,7 +56,7 @@ struct Args {
   int64_t M, N, K;       // N: rows of the B operand (both weights of a gate/up pair)
   int axis, pieces;      // 0: one piece; 1: A and B in pieces along K; 2: B and C along N; 3: A and C along M
   int64_t len[3];        // lengths of the pieces along that axis: every piece starts a tile (a k-tile) of its own
-  int tm0, tms, tns;     // first tile row of this launch, its tile rows and columns
+  int tms, tns;          // tile rows and columns of this launch
   int splits;            // K splits; > 1: fp32 partial products at part + split * M * N
   float* part;
   void* c[3];
@@ -111,7 +111,6 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
 
   int tm, tn, sp;
   work_coords(blockIdx.x, ar.tms, ar.tns, ar.splits, tm, tn, sp);
-  tm += ar.tm0;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;

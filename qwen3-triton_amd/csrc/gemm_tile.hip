@@ -71,19 +71,18 @@ int64_t tile_cols(const Args& a, int bn) {
 // combine: what the combining pass adds besides its traffic (us): a launch (4.5 measured on small products), or
 // next to nothing where the pass also forms the norm that an unsplit product would leave to a launch of its own.
 // can_split: the product may be formed as partial products (plain or residual epilogue, 16-byte columns).
-Plan plan_for(const Args& a, bool at, bool bt, bool can_split, double combine, int64_t row0 = 0) {
+Plan plan_for(const Args& a, bool at, bool bt, bool can_split, double combine) {
   Plan best{0, 1};
   double best_t = 0.0;
-  const int64_t rows = a.M - row0;
   for (int c = 0; c < kNumCfg; ++c) {
     if (!cfg_for(c, at, bt)) continue;
-    if (kCfg[c].bm >= 2 * rows && kCfg[c].bm > (bt ? 64 : 32)) continue;  // more than half of the tile's rows empty
-    const int64_t tiles = (tile_rows(a, kCfg[c].bm) - row0 / kCfg[c].bm) * tile_cols(a, kCfg[c].bn);
+    if (kCfg[c].bm >= 2 * a.M && kCfg[c].bm > (bt ? 64 : 32)) continue;  // more than half of the tile's rows empty
+    const int64_t tiles = tile_rows(a, kCfg[c].bm) * tile_cols(a, kCfg[c].bn);
     for (int sp : kSplits) {
       // a grid that fills the chip by itself is not split: its partial products would outgrow the caches
       // (6144 x 4096 x 8192 in two splits: 390 + 43 us against 300 us in two launches, below)
       if (sp > 1 && (!can_split || a.K / sp < kMinSplitK || tiles >= 256 * kCfg[c].conc)) break;
-      const double t = estimate(c, sp, tiles, rows, a.N, a.K, combine);
+      const double t = estimate(c, sp, tiles, a.M, a.N, a.K, combine);
       if (best_t == 0.0 || t < best_t) {
         best = {c, sp};
         best_t = t;
@@ -267,15 +266,23 @@ bool parse(const q3_gemm_desc* d, Call& c) {
   return tile_rows(a, 32) * tile_cols(a, 64) < (1ll << 28);
 }
 
-// rows row0 .. row1 - 1 (multiples of the tile rows, or the end)
-int launch(Call& c, const Plan& p, int64_t row0, int64_t row1, int dtype, hipStream_t s) {
-  const Cfg& f = kCfg[p.cfg];
-  c.a.tm0 = (int)(row0 / f.bm);
-  c.a.tms = (int)((row1 < c.a.M ? row1 / f.bm : tile_rows(c.a, f.bm)) - c.a.tm0);
-  c.a.tns = (int)tile_cols(c.a, f.bn);
-  if (c.at) return q3gemm::launch_tile_tn(dtype, p.cfg, c.a, s);
-  if (c.bt) return q3gemm::launch_tile_nn(dtype, p.cfg, c.epi, c.a, s);
-  return q3gemm::launch_tile_nt(dtype, p.cfg, c.epi, c.a, s);
+// One launch of a call: its arguments (the rows it forms are rows of its own operands), tiles and grid.
+struct Launch {
+  Args a;
+  Plan p;
+  int64_t rows;
+};
+
+void set_grid(Launch& l) {
+  const Cfg& f = kCfg[l.p.cfg];
+  l.a.tms = (int)(l.rows < l.a.M ? l.rows / f.bm : tile_rows(l.a, f.bm));
+  l.a.tns = (int)tile_cols(l.a, f.bn);
+}
+
+int launch(const Call& c, const Launch& l, int dtype, hipStream_t s) {
+  if (c.at) return q3gemm::launch_tile_tn(dtype, l.p.cfg, l.a, s);
+  if (c.bt) return q3gemm::launch_tile_nn(dtype, l.p.cfg, c.epi, l.a, s);
+  return q3gemm::launch_tile_nt(dtype, l.p.cfg, c.epi, l.a, s);
 }
 
 // 256 x 256 tiles whose last round leaves at least 3/8 of the CUs idle: the rows that fill whole rounds first,
@@ -290,6 +297,51 @@ int64_t whole_round_rows(const Call& c, const Plan& p) {
   return tiles / 256 * 256 / tn * 256;
 }
 
+// The call without its first rows: a call of its own, so that its tiles start at the first row left whatever
+// their height, and no row is formed twice (the residual may be the output itself).
+void drop_rows(Args& a, bool at, int64_t rows) {
+  a.M -= rows;
+  if (a.axis == 3) {
+    for (; rows >= a.len[0]; --a.pieces) {
+      rows -= a.len[0];
+      for (int i = 0; i + 1 < a.pieces; ++i) {
+        a.a.p[i] = a.a.p[i + 1];
+        a.a.ld[i] = a.a.ld[i + 1];
+        a.c[i] = a.c[i + 1];
+        a.ldc[i] = a.ldc[i + 1];
+        a.len[i] = a.len[i + 1];
+      }
+    }
+    a.len[0] -= rows;
+  }
+  for (int i = 0; i < (a.axis == 1 ? a.pieces : 1); ++i) a.a.p[i] += at ? rows : rows * a.a.ld[i];
+  for (int i = 0; i < (a.axis == 3 ? 1 : 3); ++i)  // axis 2: every piece; dg and du share dg's stride
+    if (a.c[i]) a.c[i] = (u16*)a.c[i] + rows * a.ldc[a.axis == 2 ? i : 0];
+  const int64_t out = rows * a.ldc[0], in = rows * a.ldgu;
+  if (a.res) a.res += rows * a.ldres;
+  if (a.g) a.g += out;
+  if (a.u) a.u += out;
+  if (a.gin) a.gin += in;
+  if (a.uin) a.uin += in;
+}
+
+// The launches of a call, one or two.
+int launches(const Call& c, Launch* l) {
+  l[0].a = c.a;
+  l[0].p = plan_for(c.a, c.at, c.bt, c.can_split, c.combine);
+  l[0].a.splits = l[0].p.splits;
+  const int64_t m1 = whole_round_rows(c, l[0].p);
+  l[0].rows = m1 > 0 ? m1 : c.a.M;
+  set_grid(l[0]);
+  if (m1 == 0) return 1;
+  l[1].a = c.a;
+  drop_rows(l[1].a, c.at, m1);
+  l[1].p = plan_for(l[1].a, c.at, c.bt, false, c.combine);
+  l[1].rows = l[1].a.M;
+  set_grid(l[1]);
+  return 2;
+}
+
 }  // namespace
 
 extern "C" {
@@ -301,39 +353,49 @@ size_t q3_gemm_workspace_bytes(const q3_gemm_desc* d) {
   return p.splits > 1 ? (size_t)p.splits * (size_t)c.a.M * (size_t)c.a.N * sizeof(float) : 0;
 }
 
+int q3_gemm_plan(const q3_gemm_desc* d, int64_t* out) {
+  Call c;
+  Launch l[2];
+  if (!out || !parse(d, c)) return 0;
+  const int n = launches(c, l);
+  for (int i = 0; i < n; ++i) {
+    const Cfg& f = kCfg[l[i].p.cfg];
+    const int64_t row[5] = {c.a.M - l[i].a.M, l[i].rows, f.bm, f.bn, l[i].p.splits};
+    std::copy(row, row + 5, out + 5 * i);
+  }
+  return n;
+}
+
 int q3_gemm(const q3_gemm_desc* d, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   Call c;
   Q3_REQUIRE(parse(d, c));
-  Plan p = plan_for(c.a, c.at, c.bt, c.can_split, c.combine);
+  Launch l[2];
+  const int n = launches(c, l);
   const bool norm = d->epilogue == Q3_GEMM_RESIDUAL_NORM;
-  if (p.splits > 1) {
+  if (l[0].p.splits > 1) {
+    Args& a = l[0].a;
     Q3_REQUIRE(workspace && al16(workspace) &&
-               workspace_bytes >= (size_t)p.splits * (size_t)c.a.M * (size_t)c.a.N * sizeof(float));
-    c.a.splits = p.splits;
-    c.a.part = (float*)workspace;
-    const int rc = launch(c, p, 0, c.a.M, d->dtype, stream);
+               workspace_bytes >= (size_t)a.splits * (size_t)a.M * (size_t)a.N * sizeof(float));
+    a.part = (float*)workspace;
+    const int rc = launch(c, l[0], d->dtype, stream);
     if (rc != 0) return rc;
     if (norm) {
       if (d->dtype == Q3_BF16)
-        combine_norm_kernel<BF16><<<(unsigned)c.a.M, 512, 0, stream>>>(c.a, (const u16*)d->norm_w, d->eps, (u16*)d->y, d->ldy);
+        combine_norm_kernel<BF16><<<(unsigned)a.M, 512, 0, stream>>>(a, (const u16*)d->norm_w, d->eps, (u16*)d->y, d->ldy);
       else
-        combine_norm_kernel<F16><<<(unsigned)c.a.M, 512, 0, stream>>>(c.a, (const u16*)d->norm_w, d->eps, (u16*)d->y, d->ldy);
+        combine_norm_kernel<F16><<<(unsigned)a.M, 512, 0, stream>>>(a, (const u16*)d->norm_w, d->eps, (u16*)d->y, d->ldy);
     } else {
-      const unsigned g = (unsigned)cdiv(c.a.M * (c.a.N / 8), 256);
-      if (d->dtype == Q3_BF16) combine_kernel<BF16><<<g, 256, 0, stream>>>(c.a);
-      else combine_kernel<F16><<<g, 256, 0, stream>>>(c.a);
+      const unsigned g = (unsigned)cdiv(a.M * (a.N / 8), 256);
+      if (d->dtype == Q3_BF16) combine_kernel<BF16><<<g, 256, 0, stream>>>(a);
+      else combine_kernel<F16><<<g, 256, 0, stream>>>(a);
     }
     return (int)hipGetLastError();
   }
-  const int64_t m1 = whole_round_rows(c, p);
-  if (m1 > 0) {
-    const int rc = launch(c, p, 0, m1, d->dtype, stream);
+  for (int i = 0; i < n; ++i) {
+    const int rc = launch(c, l[i], d->dtype, stream);
     if (rc != 0) return rc;
-    p = plan_for(c.a, c.at, c.bt, false, c.combine, m1);
   }
-  const int rc = launch(c, p, m1, c.a.M, d->dtype, stream);
-  if (rc != 0 || !norm) return rc;
-  return q3_rmsnorm_fwd(d->dtype, d->c[0], d->norm_w, d->y, d->m, d->n, d->eps, stream);
+  return norm ? q3_rmsnorm_fwd(d->dtype, d->c[0], d->norm_w, d->y, d->m, d->n, d->eps, stream) : 0;
 }
 
 // LM-head logits A B^T, stored, with their cross-entropy statistics (q3hip.h): 256 x 256 tiles, 128 x 256 when

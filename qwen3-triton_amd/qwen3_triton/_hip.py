@@ -113,6 +113,7 @@ SIGNATURES: dict[str, tuple] = {
     "q3_greedy_select": (_i32, [_i32, _p, _i64, _i64, _i64, _p, _p, _i64, _i64, _p, _p, _p, _p, _i32, _i64, _p]),
     "q3_advance": (_i32, [_p, _i64, _p]),
     "q3_gemm_workspace_bytes": (_sz, [_p]),
+    "q3_gemm_plan": (_i32, [_p, _p]),
     "q3_gemm": (_i32, [_p, _p, _sz, _p]),
     "q3_gemm_strided": (_i32, [_i32, _i32, _p, _i64, _i64, _p, _i64, _i64, _p, _i64, _i64, _i64, _i64, _f32, _i32,
                                 _p]),

@@ -126,6 +126,25 @@ def test_epilogues(m, n, k, dtype):
         assert torch.equal(dg, eg) and torch.equal(du, eu)
 
 
+@pytest.mark.parametrize("m,n,k", [(6145, 4096, 4096), (9300, 4096, 512), (4700, 8192, 512), (12800, 2048, 512)])
+def test_residual_in_place_over_two_launches(m, n, k):
+    """Row counts that q3_gemm forms in two launches, the second on 192-row tiles: with the residual in place no
+    row takes the product twice, and the norm is that of the same sum."""
+    print(f"q3_gemm residual in place {m}x{n}x{k}", flush=True)
+    gen = torch.Generator("cuda").manual_seed(m)
+    dt = torch.bfloat16
+    x, w, res = (torch.randn(s, generator=gen, device="cuda").to(dt) for s in ((m, k), (n, k), (m, n)))
+    nw = torch.randn(n, generator=gen, device="cuda").to(dt)
+    y, c = torch.empty_like(res), res.clone()
+    gemm([x], [w], [y], m, n, k)
+    e = _ops.add(res, y)
+    gemm([x], [w], [c], m, n, k, epilogue=H.GEMM_RESIDUAL, res=c)
+    assert torch.equal(c, e)
+    c, h = res.clone(), torch.empty_like(res)
+    gemm([x], [w], [c], m, n, k, epilogue=H.GEMM_RESIDUAL_NORM, res=c, norm=(nw, 1e-6, h))
+    assert torch.equal(c, e) and torch.equal(h, _ops.rmsnorm_fwd(e, nw, 1e-6))
+
+
 def test_refusals():
     x = torch.zeros(16, 64, device="cuda", dtype=torch.bfloat16)
     c = torch.zeros(16, 16, device="cuda", dtype=torch.bfloat16)
