@@ -2,13 +2,15 @@
 
 New here (the reference materialises [B,S,V] logits: ``qwen3_triton/_model.py:131-132``
 ``lm_head`` then ``kernels/loss.py:46-71``).  On the matrix cores one GEMM over the vocabulary forms the
-logits, keeps them in the activation dtype (bf16: the reference's own lm_head output, whose [T, V] copy
-it materialises too) and folds those stored values into per-row (max, sum-exp) partials plus the target
-logit; a final merge gives lse and the token-mean loss.  The backward turns the logits in place into
-dz = (softmax - onehot) * up / count and forms dW = dz^T . h and dX = dz . W from them as they lie, one GEMM
-each, for any token count.  Other types and widths work through chunks of ``chunk`` vocabulary columns whose
-fp32 logits live in one reusable [T, chunk] buffer and are recomputed in the backward.  The same math as
-``linear`` followed by ``causal_cross_entropy``.
+logits and folds them into per-row (max, sum-exp) partials plus the target logit; a final merge gives lse and
+the token-mean loss.  Whole 8-token groups at a ``chunk`` of whole 8-column groups also keep the logits in the
+activation dtype (bf16: the reference's own lm_head output, whose [T, V] copy it materialises too) and take the
+statistics from those stored values; the backward turns them in place into dz = (softmax - onehot) * up / count
+and forms dW = dz^T . h and dX = dz . W from them as they lie, one GEMM each (a second backward forms the consumed
+logits again).  Elsewhere the statistics and dz come from fp32 logits, which the backward recomputes: in the epilogue
+of a second logits GEMM (for token counts off that grid by chunks of ``chunk`` vocabulary columns, dX summed over
+them in fp32: no [T, V] buffer), or, for other types and widths, in one reusable fp32 [T, chunk] buffer.  The same
+math as ``linear`` followed by ``causal_cross_entropy``.
 """
 import torch
 
@@ -31,16 +33,15 @@ def _chunk_logits(x, w, c0, n, zbuf):
         matmul_into(x, w[c0:c0 + n].t(), zbuf[:, :n])
 
 
-def _stored_ok(x, w):
-    return _mfma_ok(x, w) and x.shape[-1] % 64 == 0 and gemm_ok(x, w)
+def _fused_ok(x, w):
+    """The logits GEMM's statistics and gradient epilogues, and q3_gemm over the [T, V] dz (row stride V)."""
+    return _mfma_ok(x, w) and x.shape[-1] % 64 == 0 and gemm_ok(x, w) and w.shape[0] < 1 << 22
 
 
 def _stored_logits(x, w, tgt):
-    """(statistics, logits [T, V]): one GEMM over the vocabulary whose epilogue stores the logits in the
-    activation dtype (the reference's bf16 lm_head output) and forms the statistics from them, one partial per
-    128 columns; no fp32 logits in memory, and no second logits GEMM in the backward."""
+    """(statistics, logits [T, V] in the activation dtype): the statistics are of the stored, rounded logits."""
     t, v = x.shape[0], w.shape[0]
-    st = _ops.CEState(t, -(-v // 128), x.device)
+    st = _ops.CEState(t, -(-v // 128), x.device)   # a partial per 128 columns
     z = torch.empty((t, v), device=x.device, dtype=x.dtype)
     st.gemm_stats_store(0, x, w, 0, v, tgt, z)
     return st, z
@@ -64,8 +65,12 @@ class _LMHeadCE(torch.autograd.Function):
         chunk = min(chunk, v)
         nch = -(-v // chunk)
         z = None
-        if _stored_ok(x, weight):
-            st, z = _stored_logits(x, weight, tgt)
+        if _fused_ok(x, weight):
+            if (b * s) % 8 == 0 and chunk % 8 == 0:
+                st, z = _stored_logits(x, weight, tgt)
+            else:
+                st = _ops.CEState(b * s, -(-v // 128), hidden.device)
+                st.gemm_stats(0, x, weight, 0, v, tgt)
         else:
             st = _ops.CEState(b * s, nch, hidden.device)
             zbuf = torch.empty((b * s, chunk), device=hidden.device, dtype=torch.float32)
@@ -90,11 +95,15 @@ class _LMHeadCE(torch.autograd.Function):
         dw = torch.empty_like(weight)
         mfma = _mfma_ok(x, weight) and t % 8 == 0
         z, ctx.z = ctx.z, None   # consumed: dz overwrites the stored logits in place
-        if z is None and _stored_ok(x, weight):   # a second backward of the same graph
-            z = _stored_logits(x, weight, tgt)[1]
-        if z is not None:
-            # dz from the stored logits, in place; dW = dz^T . x and dX = dz . W read it as it lies
-            _ops.ce_grad(z, v, v, 0, tgt, lse, count, up, z, v, v, ctx.ignore)
+        fused = _fused_ok(x, weight)
+        if mfma and fused:   # [T, V] dz
+            if chunk % 8:
+                z = torch.empty((t, v), device=x.device, dtype=x.dtype)
+                _ops.gemm_ce_grad(x, weight, 0, v, tgt, lse, count, up, z, v, ctx.ignore)
+            else:
+                if z is None:   # a second backward: the logits that lse was formed from, again
+                    z = _stored_logits(x, weight, tgt)[1]
+                _ops.ce_grad(z, v, v, 0, tgt, lse, count, up, z, v, v, ctx.ignore)
             dx = None
             if ctx.needs_input_grad[1]:
                 gemm([z], [x], [dw], v, h, t, kmajor=(True, True))
@@ -105,7 +114,7 @@ class _LMHeadCE(torch.autograd.Function):
                 gemm([z], [weight], [dx], t, h, v, kmajor=(False, True))
                 dx = dx.view(b, s, h)
             return dx, dw, None, None, None
-        zbuf = torch.empty((t, chunk), device=x.device, dtype=torch.float32)
+        zbuf = None if fused else torch.empty((t, chunk), device=x.device, dtype=torch.float32)
         dz = torch.empty((t, chunk), device=x.device, dtype=x.dtype)
         dx = torch.empty((t, h), device=x.device, dtype=torch.float32)
         if mfma:
@@ -114,8 +123,11 @@ class _LMHeadCE(torch.autograd.Function):
         for c in range(-(-v // chunk)):
             c0 = c * chunk
             n = min(chunk, v - c0)
-            _chunk_logits(x, weight, c0, n, zbuf)
-            _ops.ce_grad(zbuf, chunk, n, c0, tgt, lse, count, up, dz, chunk, v, ctx.ignore)
+            if fused:
+                _ops.gemm_ce_grad(x, weight, c0, n, tgt, lse, count, up, dz, v, ctx.ignore)
+            else:
+                _chunk_logits(x, weight, c0, n, zbuf)
+                _ops.ce_grad(zbuf, chunk, n, c0, tgt, lse, count, up, dz, chunk, v, ctx.ignore)
             if mfma:
                 gemm_nt_into(dz, chunk, wt[:, c0:], wt.shape[1], dx, t, h, n, accumulate=c > 0)
                 dzt = _ops.transpose_last2(dz)            # [chunk, T]

@@ -270,3 +270,24 @@ def test_lm_head_ce_second_backward_recomputes():
     for a, b in zip(g1, g2):
         assert cosine(a, b) >= 0.9999
         assert max_rel(a, b) <= 2e-2
+
+
+@pytest.mark.parametrize("b,s,chunk", [(1, 203, 16384), (3, 67, 512), (2, 52, 1001)])
+def test_lm_head_ce_keeps_fp32_logits(b, s, chunk):
+    """Token counts and chunks off the 8-element grid form loss and gradients from fp32 logits, at logits of
+    deviation 6 (a trained head's): what is left is the roundings of dz and of the gradient, at most 2^-9 of a
+    value each; logits held in bf16 in between leave 1e-2.  The forward holds no logits."""
+    print(f"lmhead fp32 logits {b} {s} {chunk}", flush=True)
+    h, v, gen = 512, 4096, seeded(b * s)
+    x0, w0 = randn(b, s, h, gen=gen, dtype=torch.bfloat16), randn(v, h, gen=gen, dtype=torch.bfloat16, scale=6 * h ** -0.5)
+    y = labels_for(b, s, v, gen).cuda()
+    x, w = x0.cuda().requires_grad_(), w0.cuda().requires_grad_()
+    before = torch.cuda.memory_allocated()
+    loss = lm_head_cross_entropy(x, w, y, chunk=chunk)
+    assert torch.cuda.memory_allocated() - before < b * s * v
+    xr, wr = x0.cuda().double().requires_grad_(), w0.cuda().double().requires_grad_()
+    z = (xr @ wr.t())[:, :-1].reshape(-1, v)
+    e = torch.nn.functional.cross_entropy(z, y[:, 1:].reshape(-1), ignore_index=-100)
+    assert abs(float(loss.detach()) - float(e.detach())) <= 1e-5 * float(e.detach())   # 512-term fp32 sums
+    for a, r in zip(torch.autograd.grad(loss, (x, w)), torch.autograd.grad(e, (xr, wr))):
+        assert float((a.double() - r).norm() / r.norm()) <= 2 ** -8
