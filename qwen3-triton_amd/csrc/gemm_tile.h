@@ -167,17 +167,19 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
     return (uint32_t)(((km ? (lane / (bd / 8)) * (bd / 8) : (lane >> 3)) * (int)ld + chk * 8) * 2);
   };
   uint32_t offa = lane_off(lda, AT, achk, BM), offb = lane_off(ldb, BT, bchk, BN);
-  // The next k-tile's descriptors, formed while the matrix cores run (prep) and used after the barrier (issue).
   constexpr int BDIV = EPI == 3 ? 2 : 1;  // gate/up: each weight holds half of the operand's rows
+  // The next k-tile's descriptors, formed while the matrix cores run (prep) and used after the barrier (issue).
+  // They span one tile's rows, so the operand itself may be of any size.
   int64_t basea = 0, baseb = 0;  // element offset of the tile in its piece
-  int rema = 0, remb = 0;        // 16-byte units from there to the piece's end
+  int rema = 0, remb = 0;        // 16-byte units: k contiguous, from there to the end of the tile's last row; K-major,
+                                 // from there to the end of the piece's part of a k-row
   int krem = 0;                  // k left in the piece
   int tleft = nk;                // k-tiles left in this split
   auto start = [&](int64_t kp, int64_t k0) {  // the cursor at k0 of a piece of kp
     basea = AT ? k0 * lda + ma : (int64_t)ma * lda + k0;
     baseb = BT ? k0 * ldb + nb : (int64_t)(nb / BDIV) * ldb + k0;
-    rema = (int)(((AT ? (kp - 1) * lda + mrows : (int64_t)(mrows - 1) * lda + kp) - basea) >> 3);
-    remb = (int)(((BT ? (kp - 1) * ldb + ncols : (int64_t)(ncols / BDIV - 1) * ldb + kp) - baseb) >> 3);
+    rema = AT ? (mrows - ma) >> 3 : (int)(((min(mrows - ma, BM) - 1) * lda + kp - k0) >> 3);
+    remb = BT ? (ncols - nb) >> 3 : (int)(((min(ncols - nb, BN) / BDIV - 1) * ldb + kp - k0) >> 3);
     krem = (int)(kp - k0);
   };
   int pi = 0;
@@ -206,20 +208,21 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_tile_kernel(Args ar) {
   rsrc_t da, db;
   uint32_t va, vb;
   auto prep = [&]() {
-    // A descriptor spans at most 2^31 - 16 bytes (tile offsets stay below that); past the last k-tile, the
-    // only place where nothing is left, it is empty.
+    // A descriptor spans at most 2^31 - 16 bytes (row strides stay below 2^22); past the last k-tile, the only
+    // place where nothing is left, it is empty.
+    const int krow = min(krem, 64) - 1;  // last k-row of the tile
     auto bytes = [&](int rem) { return tleft > 0 ? min(rem, 0x7ffffff) * 16 : 0; };
-    da = __builtin_amdgcn_make_buffer_rsrc((void*)(pa + basea), 0, bytes(rema), 0x00027000);
-    db = __builtin_amdgcn_make_buffer_rsrc((void*)(pb + baseb), 0, bytes(remb), 0x00027000);
+    const int ea = AT ? krow * (int)(lda >> 3) + rema : rema, eb = BT ? krow * (int)(ldb >> 3) + remb : remb;
+    da = __builtin_amdgcn_make_buffer_rsrc((void*)(pa + basea), 0, bytes(ea), 0x00027000);
+    db = __builtin_amdgcn_make_buffer_rsrc((void*)(pb + baseb), 0, bytes(eb), 0x00027000);
     va = !AT && achk * 8 >= krem ? kOob : offa;
     vb = !BT && bchk * 8 >= krem ? kOob : offb;
     krem -= 64;
     --tleft;
-    const int64_t sa = AT ? 64 * lda : 64, sb = BT ? 64 * ldb : 64;
-    basea += sa;
-    baseb += sb;
-    rema -= (int)(sa >> 3);
-    remb -= (int)(sb >> 3);
+    basea += AT ? 64 * lda : 64;
+    baseb += BT ? 64 * ldb : 64;
+    if (!AT) rema -= 8;
+    if (!BT) remb -= 8;
   };
   auto issue = [&](int stage) {
     char* st = lds + stage * STAGE;

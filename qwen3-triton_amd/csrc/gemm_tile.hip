@@ -181,10 +181,9 @@ struct Call {
 
 bool operand_ok(const void* p, int64_t ld, int64_t rows, int64_t k, bool kmajor) {
   // 16-byte chunks: the contiguous extent (k, or the operand's own index when K-major) and the row stride are
-  // whole chunks; tile offsets fit the 2^31-byte range of a buffer descriptor
+  // whole chunks; a tile's offsets fit the 2^31-byte range of a buffer descriptor
   const int64_t ext = kmajor ? rows : k;
-  return p && al16(p) && ld % 8 == 0 && ext % 8 == 0 && ld >= ext && ld < (1 << 22) &&
-         ((kmajor ? k : rows) * ld) / 8 < (1ll << 31);
+  return p && al16(p) && ld % 8 == 0 && ext % 8 == 0 && ld >= ext && ld < (1 << 22);
 }
 
 bool parse(const q3_gemm_desc* d, Call& c) {

@@ -42,11 +42,15 @@ def _ld(t):
     return t.stride(0) if t.shape[0] > 1 else t.shape[1]
 
 
+MAX_LD = 1 << 22   # q3_gemm's row strides stay below (32-bit offsets within a tile)
+
+
 def _operand_ok(t):
-    """``q3_gemm``'s rule for one operand: rows of whole 16-byte chunks at a 16-byte aligned stride."""
+    """``q3_gemm``'s rule for one operand: rows of whole 16-byte chunks at a 16-byte aligned stride (and few enough
+    rows that up to three such pieces, or a gate/up pair, stay within its 32-bit sizes)."""
     ld = _ld(t)
     return t.stride(1) == 1 and t.data_ptr() % 16 == 0 and ld % 8 == 0 and t.shape[1] % 8 == 0 and \
-        t.shape[1] <= ld < 1 << 22
+        t.shape[1] <= ld < MAX_LD and t.shape[0] < 1 << 28
 
 
 def gemm_ok(*operands):
@@ -308,6 +312,7 @@ def shared_input_projections(x, weights, *, optimized=False):
     are multiples of 8 share their launches, otherwise each projection is an ordinary ``linear``."""
     if len(weights) <= 3 and x.is_contiguous() and x.numel() and \
             gemm_ok(x.view(-1, x.shape[-1]), *weights) and \
-            all(w.is_contiguous() and w.ndim == 2 and w.shape[1] == x.shape[-1] and w.shape[0] % 8 == 0 for w in weights):
+            all(w.is_contiguous() and w.ndim == 2 and w.shape[1] == x.shape[-1] and w.shape[0] % 8 == 0 and
+                w.shape[0] < MAX_LD for w in weights):
         return list(_SharedInputProjections.apply(x, *weights))
     return [linear(x, w, optimized=optimized) for w in weights]

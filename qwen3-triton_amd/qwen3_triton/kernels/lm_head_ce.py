@@ -15,7 +15,7 @@ math as ``linear`` followed by ``causal_cross_entropy``.
 import torch
 
 from . import _ops
-from .linear import gemm, gemm_nt_into, gemm_ok, matmul_into
+from .linear import MAX_LD, gemm, gemm_nt_into, gemm_ok, matmul_into
 
 DEFAULT_CHUNK = 16384
 
@@ -35,7 +35,7 @@ def _chunk_logits(x, w, c0, n, zbuf):
 
 def _fused_ok(x, w):
     """The logits GEMM's statistics and gradient epilogues, and q3_gemm over the [T, V] dz (row stride V)."""
-    return _mfma_ok(x, w) and x.shape[-1] % 64 == 0 and gemm_ok(x, w) and w.shape[0] < 1 << 22
+    return _mfma_ok(x, w) and x.shape[-1] % 64 == 0 and gemm_ok(x, w) and w.shape[0] < MAX_LD
 
 
 def _stored_logits(x, w, tgt):

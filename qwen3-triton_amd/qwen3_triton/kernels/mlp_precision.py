@@ -10,7 +10,7 @@ import torch
 
 from .. import _hip as H
 from . import _ops
-from .linear import chunk_aligned, gemm, gemm_ok, linear, linear_residual, matmul, matmul_into
+from .linear import MAX_LD, chunk_aligned, gemm, gemm_ok, linear, linear_residual, matmul, matmul_into
 
 
 def _check(x, wg, wu):
@@ -30,7 +30,7 @@ def _new(like, *shape):
 
 
 def _gate_up_ok(flat, wg, wu):
-    return wg.shape[0] % 8 == 0 and gemm_ok(flat, wg, wu)
+    return wg.shape[0] % 8 == 0 and wg.shape[0] < MAX_LD and gemm_ok(flat, wg, wu)
 
 
 def _gate_up_y(x, wg, wu):
@@ -150,6 +150,7 @@ def mlp_block(x, gate_weight, up_weight, down_weight, *, optimized=False, residu
         all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
             for t in (gate_weight, up_weight, down_weight)) and \
         x.dtype in (torch.bfloat16, torch.float16) and m > 0 and n % 8 == 0 and down_weight.shape[0] % 8 == 0 and \
+        down_weight.shape[0] < MAX_LD and \
         gemm_ok(x.view(m, k), gate_weight, up_weight, down_weight)
     if residual is not None:
         ok = ok and residual.is_contiguous() and residual.dtype == x.dtype and residual.device == x.device and \

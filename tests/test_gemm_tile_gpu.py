@@ -7,7 +7,7 @@ from _util import max_rel, randn, seeded
 
 from qwen3_triton import _hip as H
 from qwen3_triton.kernels import _ops
-from qwen3_triton.kernels.linear import gemm
+from qwen3_triton.kernels.linear import gemm, matmul
 
 pytestmark = pytest.mark.gpu
 # one rounding of the fp32 sum to the storage type: half an ulp of the largest value, 2^-9 (bf16) / 2^-12 (fp16)
@@ -193,3 +193,43 @@ def test_lm_head_ragged(b, s, h, v, dtype):
     for a, c, g in zip(first, second, grads):
         assert torch.equal(a, c)
         assert max_rel(a, g) <= (2e-2 if dtype == torch.bfloat16 else 3e-3)
+
+
+def test_operands_past_2_34_elements():
+    """K-major operands whose rows span more than 2^34 elements (34 GB): the same products as from dense ones."""
+    print("q3_gemm wide operands", flush=True)
+    k, ld, m, n = 8200, 1 << 21, 72, 136
+    buf = torch.empty(k * ld, device="cuda", dtype=torch.bfloat16)
+    a, b = buf.as_strided((k, m), (ld, 1), 0), buf.as_strided((k, n), (ld, 1), 1024)
+    gen = seeded(34)
+    a0, b0 = randn(k, m, gen=gen, dtype=torch.bfloat16).cuda(), randn(k, n, gen=gen, dtype=torch.bfloat16).cuda()
+    a.copy_(a0), b.copy_(b0)
+    assert torch.equal(matmul(a.t(), b), matmul(a0.t(), b0))          # both K-major
+    x0 = randn(m, k, gen=gen, dtype=torch.bfloat16).cuda()
+    assert torch.equal(matmul(x0, b), matmul(x0, b0))                 # a k-contiguous, b K-major
+    assert max_rel(matmul(x0, b0), x0.double() @ b0.double()) < TOL[torch.bfloat16]
+
+
+def test_lm_head_logits_past_2_34_elements():
+    """LM-head training above 2^34 logits (113080 tokens of a 151936-word vocabulary): sampled rows of both
+    gradients against fp64 (logits of deviation 1: bf16 logits leave 2^-9 of a probability)."""
+    from qwen3_triton.kernels.lm_head_ce import lm_head_cross_entropy
+    t, h, v = 113080, 64, 151936
+    print(f"lm_head {t} x {h} -> {v}", flush=True)
+    gen = torch.Generator("cuda").manual_seed(1)
+    x = torch.randn(1, t, h, generator=gen, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(v, h, generator=gen, device="cuda") * h ** -0.5).bfloat16().requires_grad_()
+    y = torch.randint(0, v, (1, t), generator=gen, device="cuda")
+    dx, dw = torch.autograd.grad(lm_head_cross_entropy(x, w, y), (x, w))
+    xs, ws = x.detach()[0].float(), w.detach().float()
+    lse = torch.cat([(xs[i:i + 4096] @ ws.t()).logsumexp(1) for i in range(0, t, 4096)]).double()
+    tgt = torch.full((t,), -1, device="cuda")
+    tgt[:-1] = y[0, 1:]
+    valid = (tgt >= 0).double() / (t - 1)
+    rows, cols = torch.tensor([0, 1, 4097, t - 9, t - 2], device="cuda"), torch.tensor([0, 7, 75000, v - 1], device="cuda")
+    xd, wd = xs.double(), ws.double()
+    dz = (xd[rows] @ wd.t() - lse[rows, None]).exp()
+    dz[torch.arange(len(rows)), tgt[rows]] -= 1
+    assert max_rel(dx[0, rows], (dz * valid[rows, None]) @ wd) <= 2e-2
+    dz = (xd @ wd[cols].t() - lse[:, None]).exp() - (tgt[:, None] == cols).double()
+    assert max_rel(dw[cols], (dz * valid[:, None]).t() @ xd) <= 2e-2
