@@ -14,7 +14,7 @@ from .._model import TritonQwen3ForCausalLM
 from ..configuration import OptimizationOptions
 from ..kernels import _ops
 from ..kernels.activation import swiglu
-from ..kernels.embedding import embedding
+from ..kernels.embedding import IdRangeError, embedding
 from ..kernels.linear import gemm, gemm_ok
 from ..kernels.mlp_precision import gate_up_swiglu
 from ..kernels.residual import residual_add
@@ -200,9 +200,12 @@ class TritonQwen3Inference(nn.Module):
             # cache is untouched when it fails
             if torch.cuda.is_current_stream_capturing():
                 raise RuntimeError('token IDs cannot be validated during graph capture')
+            table = self.model.embed_tokens.weight
+            if table.shape[0] > self.config.vocab_size:   # rows past the vocabulary are no tokens
+                table = table[:self.config.vocab_size]
             try:
-                x = embedding(input_ids, self.model.embed_tokens.weight)
-            except ValueError:
+                x = embedding(input_ids, table)
+            except IdRangeError:
                 raise ValueError('Token ID outside vocabulary') from None
         pos = kernels.positions(b, s, start, self.device, start_dev)
         try:

@@ -9,6 +9,10 @@ import torch
 from . import _ops
 
 
+class IdRangeError(ValueError):
+    """An ID outside the table's rows."""
+
+
 class _Embedding(torch.autograd.Function):
     @staticmethod
     def forward(ctx, ids, weight):
@@ -25,7 +29,7 @@ class _Embedding(torch.autograd.Function):
         bad = None if capturing else torch.zeros((), dtype=torch.int32, device=ids.device)
         y = _ops.embedding_fwd(ids, weight, bad)
         if bad is not None and bool(bad.item()):
-            raise ValueError('embedding ID out of range')
+            raise IdRangeError('embedding ID out of range')
         ctx.save_for_backward(ids)
         ctx.weight_shape = weight.shape
         ctx.weight_dtype = weight.dtype

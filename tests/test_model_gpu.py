@@ -282,3 +282,24 @@ def test_decoder_layer_8b_benchmark_shape():
         worst = min(worst, (name, c), key=lambda t: t[1])
         assert c >= 0.999, f"{name}: {c}"
     print(f"B4 S2048 layer: y max-rel {rel:.3e}, worst gradient cosine {worst[1]:.6f} ({worst[0]})", flush=True)
+
+
+def test_token_id_check_names_only_bad_ids():
+    """A bad ID is refused without touching the cache, also where the table holds more rows than the vocabulary;
+    a fault of the table keeps its own message."""
+    model, params = small_model(seed=6)
+    table = params["model.embed_tokens.weight"].cuda()
+    ids = torch.randint(0, SMALL.vocab_size, (1, 5), generator=seeded(1)).cuda()
+    want = model(ids).logits
+    model.model.embed_tokens.weight = torch.nn.Parameter(torch.cat([table, table[:8]]))
+    cache = model.new_cache(1, 8)
+    for bad in (-1, SMALL.vocab_size, SMALL.vocab_size + 8):
+        wrong = ids.clone()
+        wrong[0, 2] = bad
+        with pytest.raises(ValueError, match="Token ID outside vocabulary"):
+            model(wrong, past_key_values=cache)
+        assert cache.valid and cache.length == 0
+    assert torch.equal(model(ids, past_key_values=cache).logits, want)
+    model.model.embed_tokens.weight = torch.nn.Parameter(table.t().contiguous().t())
+    with pytest.raises(ValueError, match="Contiguous"):
+        model(ids)
