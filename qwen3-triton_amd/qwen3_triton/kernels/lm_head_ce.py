@@ -92,7 +92,6 @@ class _LMHeadCE(torch.autograd.Function):
         v, t, chunk = weight.shape[0], b * s, ctx.chunk
         x = hidden.view(t, h)
         up = dy.float().contiguous()
-        dw = torch.empty_like(weight)
         mfma = _mfma_ok(x, weight) and t % 8 == 0
         z, ctx.z = ctx.z, None   # consumed: dz overwrites the stored logits in place
         fused = _fused_ok(x, weight)
@@ -104,16 +103,16 @@ class _LMHeadCE(torch.autograd.Function):
                 if z is None:   # a second backward: the logits that lse was formed from, again
                     z = _stored_logits(x, weight, tgt)[1]
                 _ops.ce_grad(z, v, v, 0, tgt, lse, count, up, z, v, v, ctx.ignore)
-            dx = None
+            dx = dw = None
             if ctx.needs_input_grad[1]:
+                dw = torch.empty_like(weight)
                 gemm([z], [x], [dw], v, h, t, kmajor=(True, True))
-            else:
-                dw = None
             if ctx.needs_input_grad[0]:
                 dx = torch.empty((t, h), device=x.device, dtype=x.dtype)
                 gemm([z], [weight], [dx], t, h, v, kmajor=(False, True))
                 dx = dx.view(b, s, h)
             return dx, dw, None, None, None
+        dw = torch.empty_like(weight)
         zbuf = None if fused else torch.empty((t, chunk), device=x.device, dtype=torch.float32)
         dz = torch.empty((t, chunk), device=x.device, dtype=x.dtype)
         dx = torch.empty((t, h), device=x.device, dtype=torch.float32)

@@ -291,3 +291,18 @@ def test_lm_head_ce_keeps_fp32_logits(b, s, chunk):
     assert abs(float(loss.detach()) - float(e.detach())) <= 1e-5 * float(e.detach())   # 512-term fp32 sums
     for a, r in zip(torch.autograd.grad(loss, (x, w)), torch.autograd.grad(e, (xr, wr))):
         assert float((a.double() - r).norm() / r.norm()) <= 2 ** -8
+
+
+def test_lm_head_ce_frozen_weight_takes_no_gradient_buffer():
+    """A frozen head: the backward's memory stays below a weight gradient's, and dX is that of the trained head."""
+    gen = seeded(5)
+    h, v = 512, 65536
+    x = randn(2, 8, h, gen=gen, dtype=torch.bfloat16).cuda().requires_grad_()
+    w = randn(v, h, gen=gen, dtype=torch.bfloat16, scale=0.05).cuda()
+    y = labels_for(2, 8, v, gen).cuda()
+    loss = lm_head_cross_entropy(x, w, y)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    (dx,) = torch.autograd.grad(loss, (x,))
+    assert torch.cuda.max_memory_allocated() - before < w.numel() * 2
+    assert torch.equal(dx, torch.autograd.grad(lm_head_cross_entropy(x, w.requires_grad_(), y), (x, w))[0])
