@@ -310,9 +310,8 @@ class _SharedInputProjections(torch.autograd.Function):
 def shared_input_projections(x, weights, *, optimized=False):
     """[X W_i^T for W_i in weights] for up to three weights; 16-bit contiguous operands whose feature counts
     are multiples of 8 share their launches, otherwise each projection is an ordinary ``linear``."""
-    if len(weights) <= 3 and x.is_contiguous() and x.numel() and \
-            gemm_ok(x.view(-1, x.shape[-1]), *weights) and \
-            all(w.is_contiguous() and w.ndim == 2 and w.shape[1] == x.shape[-1] and w.shape[0] % 8 == 0 and
-                w.shape[0] < MAX_LD for w in weights):
+    if x.ndim >= 2 and x.is_contiguous() and x.numel() and 1 <= len(weights) <= 3 and \
+            all(w.ndim == 2 and w.is_contiguous() and w.shape[1] == x.shape[-1] and w.shape[0] % 8 == 0 and
+                w.shape[0] < MAX_LD for w in weights) and gemm_ok(x.view(-1, x.shape[-1]), *weights):
         return list(_SharedInputProjections.apply(x, *weights))
     return [linear(x, w, optimized=optimized) for w in weights]

@@ -145,8 +145,8 @@ def mlp_block(x, gate_weight, up_weight, down_weight, *, optimized=False, residu
     the matrix-core epilogue (16-bit contiguous operands, feature counts multiples of 8); otherwise
     exactly that composition."""
     m, k, n = x.numel() // x.shape[-1], x.shape[-1], gate_weight.shape[0]
-    ok = x.is_cuda and x.is_contiguous() and down_weight.ndim == 2 and down_weight.shape[1] == n and \
-        gate_weight.shape == up_weight.shape and gate_weight.shape[1] == k and \
+    ok = x.is_cuda and x.ndim >= 2 and x.is_contiguous() and gate_weight.ndim == down_weight.ndim == 2 and \
+        down_weight.shape[1] == n and gate_weight.shape == up_weight.shape and gate_weight.shape[1] == k and \
         all(t.dtype == x.dtype and t.device == x.device and t.is_contiguous()
             for t in (gate_weight, up_weight, down_weight)) and \
         x.dtype in (torch.bfloat16, torch.float16) and m > 0 and n % 8 == 0 and down_weight.shape[0] % 8 == 0 and \

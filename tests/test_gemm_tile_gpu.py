@@ -169,6 +169,22 @@ def test_refusals():
         H.call("q3_gemm", ctypes.addressof(d), ws.data_ptr(), need - 16, H.stream())
 
 
+def test_fused_layers_refuse_what_the_layers_refuse():
+    """A feature vector without a token axis and weights that are no matrices: the errors of ``linear`` and
+    ``gate_up_swiglu``."""
+    from qwen3_triton.kernels.linear import shared_input_projections
+    from qwen3_triton.kernels.mlp_precision import mlp_block
+    x = torch.zeros(2, 64, device="cuda", dtype=torch.bfloat16)
+    w = torch.zeros(64, 64, device="cuda", dtype=torch.bfloat16)
+    for xs, ws in ((x[0], [w, w]), (x, [w[0]]), (x, [w, w[..., None]])):
+        with pytest.raises(ValueError, match="Expected"):
+            shared_input_projections(xs, ws)
+    assert shared_input_projections(x, []) == []
+    for xs, ws in ((x[0], (w, w, w)), (x, (w[0], w[0], w)), (x, (w[..., None], w[..., None], w)), (x, (w, w, w[0]))):
+        with pytest.raises(ValueError, match="Expected"):
+            mlp_block(xs, *ws)
+
+
 @pytest.mark.parametrize("b,s,h,v", [(1, 2, 64, 8), (1, 129, 64, 264), (3, 67, 128, 1000), (1, 257, 64, 520)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_lm_head_ragged(b, s, h, v, dtype):
