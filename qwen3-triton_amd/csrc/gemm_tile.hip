@@ -39,11 +39,12 @@ struct Plan {
 
 // Estimated time of a configuration (us): whole rounds of resident workgroups at the full rate, a last round
 // that takes at least a lone workgroup's time, no less than the B operand streamed once at 6 TB/s, and for a K
-// split the partial products written and combined.  The constants are a fit to 5000 timings on MI355X (k
-// contiguous / K-major operands, M 17-4096, N 1024-24576, K 64-24576); the plan it picks is 2 % slower on
-// average than the best of the measured configurations and splits, 32 % at worst (1000 x 1024 x 1024).  The
-// order matters more than the values: 256 x 256 tiles sustain 1.38-1.45 PFLOP/s once they fill the CUs, smaller
-// tiles and splits keep the CUs busy below that (65 x 4096 x 4096: 15 us against 47 us on 32 tiles of 128 x 128).
+// split the partial products written and combined.  The constants are a fit to timings on MI355X; measured again
+// over 225 shapes (k contiguous / K-major operands, M 17-4096, N 1024-24576, K 64-12288; 4063 timings) the plan it
+// picks is 1.7 % slower on average than the best of all configurations and splits, 7 % at the 90th percentile, 26 %
+// at worst (512 x 1024 x 1024: 8.3 against 6.6 us).  The order matters more than the values: 256 x 256 tiles sustain
+// 1.38-1.45 PFLOP/s once they fill the CUs, smaller tiles and splits keep the CUs busy below that (65 x 4096 x 4096:
+// 15 us against 47 us on 32 tiles of 128 x 128).
 double estimate(int c, int splits, int64_t tiles, int64_t M, int64_t N, int64_t K, double combine) {
   const Cfg& f = kCfg[c];
   const int64_t w = tiles * splits, slots = 256 * f.conc;

@@ -106,6 +106,8 @@ def gemm_nt_into(a, lda, bnk, ldb, out, m, n, k, *, alpha=1.0, accumulate=False)
            out.data_ptr(), out.stride(0), m, n, k, float(alpha), int(accumulate), H.stream())
 
 
+# Launchers of the C entries for full tiles (k-contiguous operands); the modules launch ``gemm``.
+
 def gate_up_swiglu_into(x, wg, wu, g, u, y, m, n, k):
     """g = x wg^T, u = x wu^T, y = silu(g) * u in one matrix-core GEMM (M % 256 == 0, N % 128 == 0,
     K % 64 == 0; contiguous [M, K] x and [N, K] weights, contiguous [M, N] outputs); g and u None:
